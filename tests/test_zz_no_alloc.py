@@ -122,8 +122,8 @@ def test_score_noalloc_two_contexts_share_then_refuse_overlap():
             assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
         # overlapping: a's call is queued behind the products, b's is refused
         a.set_stream(busy.cuda_stream)
+        got_a, got_b = out(), out()  # before the products: out() waits for the device
         occupy()
-        got_a, got_b = out(), out()
         a.score_noalloc(ha, q.data_ptr(), kv.TYPE_BF16, Tq, HQ, HKV, D, got_a.data_ptr())
         with pytest.raises(kv.KvMemError) as ex:
             b.score_noalloc(hb, q.data_ptr(), kv.TYPE_BF16, Tq, HQ, HKV, D, got_b.data_ptr())
