@@ -7,29 +7,40 @@
 // GEMM (rows x 128 keys x head_dim) whose output is reduced by max at once,
 // so no score ever goes to memory.
 //
-// Mapping.  A workgroup of 4 waves (one per SIMD) owns one (layer, KV head,
-// 384-row slice) and a contiguous range of blocks; two workgroups share a
-// CU, so each SIMD runs two waves that cover each other's barrier and
-// load waits.  Each wave keeps 96 query rows resident in VGPRs as f16
-// A-fragments of v_mfma_f32_16x16x32_f16 (loaded once; bf16 queries are
-// converted to f16 on the way, exact for normal-range values, a wave's rows
-// scaled by a power of two first when they would overflow f16), so every
-// 16-byte B-fragment read from LDS feeds six MFMAs (two reads kept in
-// flight ahead of their MFMAs).  Half a block's K tile
-// (64 keys x head_dim halves of one KV head, 32 KiB) moves HBM -> LDS with
-// global_load_lds_dwordx4 (no register staging) into one of two LDS
-// buffers while the other buffer's keys are multiplied: one barrier per
-// half block.  The per-block max over the wave's lanes uses DPP and the
-// row-swap permutes, not LDS.  Inside a tile the
-// 16-byte chunk c of key j sits at chunk position c ^ (j mod chunks-per-
-// key), so the 16 keys of a B-fragment read hit 16 different bank groups;
-// the swizzle is applied on the global side (each lane of a direct LDS load
-// fetches the chunk that belongs to its fixed LDS slot).  Out-of-range
-// query rows and keys (partial last block, row count not a multiple of
-// 384) are replaced by duplicates of valid ones, which leaves the max
-// unchanged and needs no masking.  Each wave writes its own per-block max
-// to a partial array; a small kernel folds waves, row slices, KV heads and
-// layers.
+// Mapping.  A workgroup owns one (layer, KV head, row slice) and a contiguous
+// range of blocks.  Its 1, 2 or 4 waves hold up to 6 tiles of 16 query rows
+// each, resident in VGPRs as f16 A-fragments of v_mfma_f32_16x16x32_f16
+// (loaded once; bf16 queries are converted to f16 on the way, exact for
+// normal-range values, a wave's rows scaled by a power of two when they would
+// overflow f16), so every 16-byte B-fragment read from LDS feeds as many
+// MFMAs as the wave has tiles (two reads kept in flight ahead of their
+// MFMAs).  The key tile (16 keys per wave of the workgroup) moves HBM -> LDS
+// with global_load_lds_dwordx4 (no register staging) into one of two LDS
+// buffers while the other's keys are multiplied.
+//  - Up to 96 rows fit one wave: it streams its keys alone, without a
+//    barrier, the next tile's loads always in flight.  HBM-bound: 14 query
+//    tokens of 24 heads over 16 x 2048 blocks read 8.59 GB in 1.22 ms = 7.0
+//    TB/s, the rate of a plain read (2.03 ms when every slice was padded to
+//    the 384 rows of four waves).
+//  - More rows go to two or four waves that share each key tile, one barrier
+//    per tile; with four waves of 6 tiles the matrix pipes and the power cap
+//    bound it.  384 rows make a slice; more rows make equal slices.
+//  - A block's keys are a run of 16-key groups and a tile may hold groups of
+//    several blocks, so blocks of 16, 32 or 64 keys cost no padding (16 x
+//    4096 blocks of 32 keys, 64-token query: 1.26 ms; 4.35 when every block
+//    took two tiles of 64 keys).
+//  - A launch of few blocks splits each block's keys over up to four waves'
+//    workgroups.
+// The per-block max over a wave's lanes uses DPP and the row-swap permutes,
+// not LDS.  Inside a tile the 16-byte chunk c of key j sits at chunk position
+// c ^ (j mod chunks-per-key), so the 16 keys of a B-fragment read hit 16
+// different bank groups; the swizzle is applied on the global side (each lane
+// of a direct LDS load fetches the chunk that belongs to its fixed LDS slot).
+// Out-of-range query rows and keys (partial last block, a block length or row
+// count that is no multiple of 16) are replaced by duplicates of valid ones,
+// which leaves the max unchanged and needs no masking.  Each wave writes its
+// own per-block max to a partial array; a small kernel folds waves, key parts,
+// row slices, KV heads and layers.
 //
 // The file is built with finite-math semantics (max needs no NaN
 // canonicalisation); every identity is -FLT_MAX and inputs are finite F16.
@@ -52,25 +63,39 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-constexpr int kScoreWaves = 4;
-constexpr int kScoreThreads = kScoreWaves * 64;
-constexpr int kRowTiles = 6;                               // 16-row tiles per wave
-constexpr int kRowsPerWave = kRowTiles * 16;               // 96
-constexpr int kRowsPerGroup = kScoreWaves * kRowsPerWave;  // 384
-constexpr int kMaxTokens = 128;                            // keys per block (at most)
-constexpr int kTileKeys = 64;                              // keys per LDS tile (half a block)
-// Cache policy of the tile DMA: nt (streamed once; keeps L2 for the query
-// rows, and costs less energy in the power-capped regime this kernel runs in).
+constexpr int kMaxTokens = 128;  // keys per block (at most)
+// Most row tiles (of 16 query rows) a wave keeps, and waves that share a key
+// tile: a row slice is at most 24 tiles = 384 rows.  Six tiles of 256-wide
+// rows take 192 of the 256 registers that two waves per SIMD leave a wave.
+constexpr int kMaxRowTiles = 6;
+constexpr int kMaxRowWaves = 4;
+constexpr uint32_t kSliceTiles = kMaxRowTiles * kMaxRowWaves;
+constexpr uint32_t kSliceRows = kSliceTiles * 16u;
+// Below this many waves in a launch, blocks are split over key parts: 2
+// layers x 12 blocks take 8.4 us with 384 waves, 10.7 with 96; at 480 waves a
+// split already loses (12.2 against 12.7 us), to the query rows that each
+// further wave loads.
+constexpr uint32_t kSplitWaves = 256;
+// Cache policy of the tile DMA.  Keys read by one workgroup only stream past
+// the caches (nt): L2 stays with the query rows, and the power-capped kernel
+// pays less energy (16 x 2048 blocks, 64-token query: 2.404 ms against 2.435
+// with the default policy).  Where several row slices read the same keys,
+// the default policy keeps a tile in L2 for the slice that comes to it later
+// (512-token query over 16 x 8192 blocks: 69.2 ms with nt, 65.3 without).
+constexpr int kDmaDefault = 0;
 constexpr int kDmaNonTemporal = 2;
 
 struct ScoreParams {
     const uint16_t *q;       // [L][Tq][Hq][D] bf16 or f16 bits
     const uint8_t *k;        // [L][cap][T][Hkv][D] f16
-    float *partial;          // [RG * kScoreWaves][L][Hkv][B]
+    float *partial;          // [RG * KS * WR][L][Hkv][B]
     uint32_t L, Tq, Hq, Hkv, B, T, last_T, g, R, RG;
+    uint32_t KS;             // key parts of a block, a workgroup each
+    uint32_t gpb;            // 16-key groups of one key part
     uint32_t cap;            // blocks per layer in memory (>= B)
-    uint32_t n_chunks;       // block chunks per (l, h, row slice)
+    uint32_t n_chunks;       // block chunks per (l, h, row slice, key part)
     uint32_t blocks_per_chunk;
+    uint32_t slice_rows;     // query rows per slice (RT * 16 * WR)
     uint32_t q_bf16;
     uint32_t xcd_major;      // 1 if (L*Hkv) % 8 == 0
     float scale;             // 1/sqrt(D)
@@ -98,66 +123,83 @@ __device__ inline float wave_max(float m) {
     return __builtin_fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
 }
 
-// A bf16 value (its bits in the top half of `f32_bits`, the rest zero) ->
-// f16, times qscale (a power of two, exact) before the rounding.
-__device__ inline _Float16 bf16_to_half(uint32_t f32_bits, float qscale) {
-    return static_cast<_Float16>(__uint_as_float(f32_bits) * qscale);
-}
-
 // A wave's query rows as raw 16-bit A fragments (bf16 or f16 bits, not yet
-// converted).  Returns the largest |q| bit pattern the lane loaded.
-template <int D, int KS>
-__device__ __forceinline__ uint32_t load_query_bits(const ScoreParams &p, half8_t (&a)[kRowTiles][KS],
-                                                    uint32_t l, uint32_t h, uint32_t rg, uint32_t wave,
-                                                    uint32_t lrow, uint32_t kgrp) {
-    uint32_t mx = 0;
+// converted).
+template <int RT, int KS, int D>
+__device__ __forceinline__ void load_query_bits(const ScoreParams &p, half8_t (&a)[RT][KS], uint32_t l,
+                                                uint32_t h, uint32_t row0, uint32_t lrow, uint32_t kgrp) {
 #pragma unroll
-    for (int rt = 0; rt < kRowTiles; ++rt) {
-        uint32_t r = rg * kRowsPerGroup + wave * kRowsPerWave + rt * 16 + lrow;
-        r = min(r, p.R - 1u);                       // duplicate the last valid row
+    for (int rt = 0; rt < RT; ++rt) {
+        const uint32_t r = min(row0 + rt * 16u + lrow, p.R - 1u);  // duplicate the last valid row
         const uint32_t t = r / p.g;
         const uint32_t hq = h * p.g + (r - t * p.g);
         const uint16_t *qrow = p.q + ((static_cast<uint64_t>(l) * p.Tq + t) * p.Hq + hq) * D;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            const u32x4_t w = *reinterpret_cast<const u32x4_t *>(qrow + ks * 32 + kgrp * 8);
+            a[rt][ks] = __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4_t *>(qrow + ks * 32 + kgrp * 8));
+        }
+    }
+}
+
+// Raw bf16 A fragments -> f16 in place, times qscale (a power of two, exact)
+// before the rounding.  Returns the largest |q| the lane converted.
+template <int RT, int KS, bool SCALED>
+__device__ __forceinline__ float convert_query_bits(half8_t (&a)[RT][KS], float qscale) {
+    float mx = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                mx = max(mx, max(w[i] & 0x7fffu, (w[i] >> 16) & 0x7fffu));
+    for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const u32x4_t w = __builtin_bit_cast(u32x4_t, a[rt][ks]);
+            half8_t v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {  // two bf16 per word, the low one first
+                const float lo = __uint_as_float(w[i] << 16);
+                const float hi = __uint_as_float(w[i] & 0xffff0000u);
+                mx = __builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
+                v[2 * i] = static_cast<_Float16>(SCALED ? lo * qscale : lo);
+                v[2 * i + 1] = static_cast<_Float16>(SCALED ? hi * qscale : hi);
             }
-            a[rt][ks] = __builtin_bit_cast(half8_t, w);
+            a[rt][ks] = v;
         }
     }
     return mx;
 }
 
-template <int D>
-__global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) {
+// Waves per SIMD a kernel is built for: its A fragments take RT * D / 8 of
+// a wave's registers, about 45 go to the rest.
+__host__ __device__ constexpr int score_occupancy(int D, int RT) {
+    return RT * D >= 4 * 256 ? 2 : RT * D >= 6 * 128 ? 3 : 4;
+}
+
+template <int D, int RT, int WR, bool SEG, bool REUSE>
+__global__ __launch_bounds__(WR * 64, score_occupancy(D, RT)) void score_kernel(ScoreParams p) {
     constexpr int KS = D / 32;                       // k-steps of 32
     constexpr int ROW_BYTES = D * 2;                 // one key of one head
     constexpr int CH = D / 8;                        // 16-byte chunks per key
-    constexpr int TILE = kTileKeys * ROW_BYTES;      // 32 KiB (D = 256)
-    constexpr int LOADS = TILE / 1024;               // wave-wide 1 KiB loads per tile
-    constexpr int LOADS_PER_WAVE = LOADS / kScoreWaves;
-    static_assert(LOADS % kScoreWaves == 0, "tile must split over the waves");
+    constexpr int GROUP = 16 * ROW_BYTES;            // 16 keys: 8 KiB (D = 256)
+    constexpr int TILE = WR * GROUP;                 // a group per wave
+    constexpr int LOADS = GROUP / 1024;              // wave-wide 1 KiB loads of a group
+    constexpr int DMA = REUSE ? kDmaDefault : kDmaNonTemporal;
 
     __shared__ __attribute__((aligned(1024))) uint8_t tiles[2][TILE];
 
-    // ---- decode (layer, head, row slice, chunk) from the workgroup id
+    // ---- decode (layer, head, row slice, key part, chunk) from the workgroup id
     const uint32_t pairs = p.L * p.Hkv;
-    uint32_t lh, chunk, rg;
+    const uint32_t n_sub = p.RG * p.KS;
+    uint32_t lh, chunk, sub;
     {
         const uint32_t i = blockIdx.x;
         if (p.xcd_major) {
             const uint32_t xcd = i & 7u;
             const uint32_t local = i >> 3;
-            rg = local % p.RG;
-            const uint32_t rest = local / p.RG;
+            sub = local % n_sub;
+            const uint32_t rest = local / n_sub;
             chunk = rest % p.n_chunks;
             lh = (rest / p.n_chunks) * 8u + xcd;
         } else {
-            rg = i % p.RG;
-            const uint32_t rest = i / p.RG;
+            sub = i % n_sub;
+            const uint32_t rest = i / n_sub;
             chunk = rest % p.n_chunks;
             lh = rest / p.n_chunks;
         }
@@ -165,6 +207,8 @@ __global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) 
     if (lh >= pairs) {
         return;
     }
+    const uint32_t rg = sub / p.KS;
+    const uint32_t part = sub - rg * p.KS;
     const uint32_t l = lh / p.Hkv;
     const uint32_t h = lh - l * p.Hkv;
     const uint32_t b_begin = chunk * p.blocks_per_chunk;
@@ -174,93 +218,113 @@ __global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) 
     }
 
     const uint32_t tid = threadIdx.x;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wave = WR == 1 ? 0u : __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lane = tid & 63u;
     const uint32_t lrow = lane & 15u;   // row (A) / key (B) within a 16-tile
     const uint32_t kgrp = lane >> 4;    // which 8 of the 32 k-values
 
-    // ---- K tiles: direct HBM -> LDS, swizzled chunk order
+    // ---- K tiles: direct HBM -> LDS, swizzled chunk order.  The keys of the
+    // chunk's blocks (of this key part) are a run of 16-key groups; tile `it`
+    // holds groups [it*WR, it*WR + WR), and wave w loads group w of it, group
+    // `lg` of block `lb` (advanced by WR groups per tile).
     const uint64_t key_stride = static_cast<uint64_t>(p.Hkv) * ROW_BYTES;
-    // A full tile (64 keys inside the block) has no duplicated keys: the
-    // source offset of load `inst` (key j = KPI*inst + lane/CH, chunk
-    // (lane mod CH) ^ (j mod CH)) splits into a uniform part in SGPRs,
-    // KPI*inst*key_stride, and a per-lane part XOR a per-load constant:
-    //   lane_src ^ ((KPI*inst mod CH) * 16),
+    const uint32_t gpb = p.gpb;
+    const uint32_t key0 = part * gpb * 16u;  // the key part's first key in a block
+    const uint8_t *layer_base =
+        p.k + static_cast<uint64_t>(l) * p.cap * p.T * key_stride + static_cast<uint64_t>(h) * ROW_BYTES;
+    // A full group has no duplicated keys: the source offset of load `i` (key
+    // j = 16*w + KPI*i + lane/CH of the tile, chunk (lane mod CH) ^ (j mod
+    // CH)) splits into a uniform part in SGPRs, KPI*i*key_stride, and a
+    // per-lane part XOR a per-load constant:
+    //   lane_src ^ (((16*w + KPI*i) mod CH) * 16),
     //   lane_src = (lane/CH)*key_stride + ((lane mod CH) ^ (lane/CH))*16
     // (the XORed bits lie below ROW_BYTES, and key_stride is a multiple of
-    // it), one VALU per load.  The last tile of a partial block takes the
-    // general path, which clamps keys to the last valid one.
+    // it), one VALU per load.  A group past the last key of a partial block
+    // (or of a block length that is no multiple of 16) takes the general
+    // path, which clamps keys to the last valid one.
     constexpr uint32_t KPI = 1024u / ROW_BYTES;  // keys per wave-wide 1 KiB load
     const uint32_t lane_src = (lane / CH) * static_cast<uint32_t>(key_stride) +
                               (((lane % CH) ^ (lane / CH)) * 16u);
-    // tile `it` = keys [64*(it&1), 64*(it&1) + 64) of block b_begin + it/2
-    auto issue_tile = [&](uint32_t it, int buf) {
-        const uint32_t b = b_begin + (it >> 1);
-        const uint32_t k0 = (it & 1u) * kTileKeys;
-        const uint8_t *base = p.k + ((static_cast<uint64_t>(l) * p.cap + b) * p.T) * key_stride +
-                              static_cast<uint64_t>(h) * ROW_BYTES;
+    uint32_t lb = b_begin, lg = wave;
+    auto wrap_group = [&]() {
+        if constexpr (SEG || WR == 1) {
+            while (lg >= gpb) {
+                lg -= gpb;
+                ++lb;
+            }
+        } else if (lg >= gpb) {  // a block part is a whole number of tiles
+            lg -= gpb;
+            ++lb;
+        }
+    };
+    wrap_group();
+    auto issue_tile = [&](uint32_t buf) {
+        // a group past the chunk's end (the last tile) repeats valid keys;
+        // its maxima are never written
+        const uint32_t b = SEG ? min(lb, b_end - 1u) : lb;
+        const uint32_t k0 = key0 + lg * 16u;
+        const uint8_t *base = layer_base + static_cast<uint64_t>(b) * p.T * key_stride;
         const uint32_t nt = (b + 1 == p.B && p.last_T != 0) ? p.last_T : p.T;
+        uint8_t *dst = &tiles[buf][wave * GROUP];
         // the lane terms pass through an empty asm so the per-load offsets
         // are recomputed here (a VALU or a few per load) instead of being
-        // kept live across the loop next to the 192 registers of query rows
-        if (k0 + kTileKeys <= nt) {
+        // kept live across the loop next to the registers of query rows
+        if (k0 + 16u <= nt) {
             uint32_t ls = lane_src;
             asm volatile("" : "+v"(ls));
             const uint8_t *tbase = base + static_cast<uint64_t>(k0) * key_stride;
 #pragma unroll
-            for (int i = 0; i < LOADS_PER_WAVE; ++i) {
-                const uint32_t inst = wave * LOADS_PER_WAVE + i;
-                const uint32_t voff = ls ^ (((KPI * inst) & (CH - 1u)) * 16u);
-                const uint8_t *src = tbase + static_cast<uint64_t>(KPI * inst) * key_stride + voff;
-                __builtin_amdgcn_global_load_lds(
-                    src, (lds_void_t *) (&tiles[buf][inst * 1024u]), 16, 0, kDmaNonTemporal);
+            for (int i = 0; i < LOADS; ++i) {
+                const uint32_t voff = ls ^ (((wave * 16u + KPI * i) & (CH - 1u)) * 16u);
+                const uint8_t *src = tbase + static_cast<uint64_t>(KPI * i) * key_stride + voff;
+                __builtin_amdgcn_global_load_lds(src, (lds_void_t *) (dst + i * 1024), 16, 0, DMA);
             }
-            return;
-        }
-        uint32_t ln = lane;
-        asm volatile("" : "+v"(ln));
+        } else {
+            uint32_t ln = lane;
+            asm volatile("" : "+v"(ln));
 #pragma unroll
-        for (int i = 0; i < LOADS_PER_WAVE; ++i) {
-            const uint32_t inst = wave * LOADS_PER_WAVE + i;
-            const uint32_t slot = inst * 64u + ln;              // 16-byte LDS slot
-            const uint32_t j = slot / CH;                       // key within the tile
-            const uint32_t c = (slot % CH) ^ (j % CH);          // global chunk held there
-            const uint32_t jj = min(k0 + j, nt - 1u);           // duplicate the last key
-            const uint8_t *src = base + jj * key_stride + c * 16u;
-            __builtin_amdgcn_global_load_lds(
-                src, (lds_void_t *) (&tiles[buf][inst * 1024u]), 16, 0, kDmaNonTemporal);
+            for (int i = 0; i < LOADS; ++i) {
+                const uint32_t jg = KPI * i + ln / CH;                      // key within the group
+                const uint32_t c = (ln % CH) ^ ((wave * 16u + jg) % CH);    // global chunk held there
+                const uint32_t jj = min(k0 + jg, nt - 1u);                  // duplicate the last key
+                const uint8_t *src = base + jj * key_stride + c * 16u;
+                __builtin_amdgcn_global_load_lds(src, (lds_void_t *) (dst + i * 1024), 16, 0, DMA);
+            }
         }
+        lg += WR;
+        wrap_group();
     };
 
-    issue_tile(0u, 0);
+    const uint32_t n_tiles = ((b_end - b_begin) * gpb + WR - 1u) / WR;
+    issue_tile(0u);
+    if (WR == 1 && n_tiles > 1u) {
+        issue_tile(1u);
+    }
 
-    // ---- query rows -> A fragments (resident for the whole workgroup).  The
-    // raw bits are loaded first; bf16 rows are then converted to f16 in
-    // place.  A bf16 value past f16's range (|q| >= 65536, bf16 exponent
-    // >= 143) would turn infinite, so the wave's rows are converted times
-    // 2^-qexp, which brings its largest |q| below 65536, and its maxima are
-    // scaled back on the way out.  Both scalings are exact (qexp is 0 for
-    // rows in range), so scores do not change.
-    half8_t a[kRowTiles][KS];
-    const uint32_t qmax = load_query_bits<D, KS>(p, a, l, h, rg, wave, lrow, kgrp);
+    // ---- query rows -> A fragments (resident for the whole workgroup).
+    // bf16 rows are converted to f16 as they come.  A bf16 value past f16's
+    // range (|q| >= 65536, bf16 exponent >= 143) turns infinite there: then
+    // the wave's rows are loaded again and converted times 2^-qexp, which
+    // brings its largest |q| below 65536, and its maxima are scaled back on
+    // the way out.  Both scalings are exact, so scores do not change.
+    // Finding the largest |q| along the way, and only then the scale, takes
+    // four VALU instructions per two elements where a pass for the maximum
+    // and a scaled conversion took eight: start-up is VALU-bound, and every
+    // workgroup pays it.
+    half8_t a[RT][KS];
+    const uint32_t row0 = rg * p.slice_rows + wave * (RT * 16u);
+    load_query_bits<RT, KS, D>(p, a, l, h, row0, lrow, kgrp);
     int qexp = 0;
     if (p.q_bf16 != 0) {
-        const uint32_t e = static_cast<uint32_t>(wave_max(static_cast<float>(qmax))) >> 7;
-        qexp = (e > 142u && e < 255u) ? static_cast<int>(e) - 142 : 0;
-        const float qscale = __builtin_ldexpf(1.0f, -qexp);
-#pragma unroll
-        for (int rt = 0; rt < kRowTiles; ++rt) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const u32x4_t w = __builtin_bit_cast(u32x4_t, a[rt][ks]);
-                half8_t v;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {  // two bf16 per word, the low one first
-                    v[2 * i] = bf16_to_half(w[i] << 16, qscale);
-                    v[2 * i + 1] = bf16_to_half(w[i] & 0xffff0000u, qscale);
-                }
-                a[rt][ks] = v;
-            }
+        const float qmax = wave_max(convert_query_bits<RT, KS, false>(a, 1.0f));
+        const uint32_t e = __float_as_uint(qmax) >> 23;
+        if (e > 142u && e < 255u) {
+            qexp = static_cast<int>(e) - 142;
+            // loaded anew: the raw bits must not stay live beside the fragments
+            uint32_t again = row0;
+            asm volatile("" : "+s"(again) :: "memory");
+            load_query_bits<RT, KS, D>(p, a, l, h, again, lrow, kgrp);
+            (void) convert_query_bits<RT, KS, true>(a, __builtin_ldexpf(1.0f, -qexp));
         }
     }
     const float out_scale = __builtin_ldexpf(p.scale, qexp);
@@ -274,28 +338,48 @@ __global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) 
     const uint32_t lds0 = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) uint8_t *)(&tiles[0][0]));
     const uint32_t lane_b = lrow * ROW_BYTES + ((kgrp ^ lrow) * 16u);
 
-    float *out = p.partial +
-                 ((static_cast<uint64_t>(rg * kScoreWaves + wave) * p.L + l) * p.Hkv + h) * p.B;
-    const uint32_t n_tiles = 2u * (b_end - b_begin);
+    float *out = p.partial + ((static_cast<uint64_t>(sub * WR + wave) * p.L + l) * p.Hkv + h) * p.B;
     float m = -FLT_MAX;
+    uint32_t cb = b_begin, cg = 0;  // the block and the groups of it in m
+    auto flush = [&]() {
+        m = wave_max(m);
+        if (lane == 0) {
+            out[cb] = m * out_scale;
+        }
+        m = -FLT_MAX;
+        cg = 0;
+        ++cb;
+    };
     for (uint32_t it = 0; it < n_tiles; ++it) {
-        const int buf = static_cast<int>(it & 1u);
-        // this thread's loads of tile it have landed; after the barrier every
-        // thread's have, and every wave is done reading the other buffer
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (it + 1 < n_tiles) {
-            issue_tile(it + 1, buf ^ 1);
+        const uint32_t buf = it & 1u;
+        // this wave's loads of tile `it` have landed.  Alone, a wave keeps
+        // the next tile's loads in flight past the wait and refills a buffer
+        // as soon as it has read it; waves that share the tile meet at a
+        // barrier, after which every wave's loads have landed and every wave
+        // is done reading the other buffer.
+        if (WR > 1 || it + 1u == n_tiles) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else if (LOADS == 8) {
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else {
+            static_assert(LOADS == 8 || LOADS == 4, "loads of a group");
+            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        }
+        if constexpr (WR > 1) {
+            __syncthreads();
+            if (it + 1u < n_tiles) {
+                issue_tile(buf ^ 1u);
+            }
         }
         // B fragments of the tile: f = kt * KS + ks covers keys kt*16 .. +16
         // and k-slice ks.  The reads are inline asm with explicit
         // lgkmcnt waits that carry the fragment register as an operand:
-        // two reads stay in flight ahead of the six MFMAs that consume a
+        // two reads stay in flight ahead of the RT MFMAs that consume a
         // fragment, in three registers.  (Compiler-issued reads ended up
         // with a single register, each read waiting out the MFMAs before
         // it and its own latency after.)  Every read is waited for inside
         // the tile, before the next barrier.
-        uint32_t tb = lds0 + static_cast<uint32_t>(buf) * TILE + lane_b;
+        uint32_t tb = lds0 + buf * TILE + lane_b;
         asm volatile("" : "+v"(tb));  // recompute the read addresses per tile
         auto read_b = [&](int f) {
             const uint32_t kt = static_cast<uint32_t>(f / KS);
@@ -305,14 +389,14 @@ __global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) 
             asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr) : "memory");
             return r;
         };
-        constexpr int NF = (kTileKeys / 16) * KS;
+        constexpr int NF = WR * KS;
         constexpr int PF = 2;  // reads in flight ahead of the consumed one
         half8_t bq[PF + 1];
 #pragma unroll
         for (int f = 0; f < PF; ++f) {
             bq[f] = read_b(f);
         }
-        float4_t acc[kRowTiles];
+        float4_t acc[RT];
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             const int ks = f % KS;
@@ -331,24 +415,34 @@ __global__ __launch_bounds__(kScoreThreads, 2) void score_kernel(ScoreParams p) 
                 asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(bf) :: "memory");
             }
 #pragma unroll
-            for (int rt = 0; rt < kRowTiles; ++rt) {
+            for (int rt = 0; rt < RT; ++rt) {
                 acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     a[rt][ks], bf, ks == 0 ? float4_t{0.0f, 0.0f, 0.0f, 0.0f} : acc[rt], 0, 0, 0);
             }
             if (ks == KS - 1) {
 #pragma unroll
-                for (int rt = 0; rt < kRowTiles; ++rt) {
+                for (int rt = 0; rt < RT; ++rt) {
                     m = __builtin_fmaxf(m, __builtin_fmaxf(__builtin_fmaxf(acc[rt][0], acc[rt][1]),
                                                            __builtin_fmaxf(acc[rt][2], acc[rt][3])));
                 }
+                if constexpr (SEG) {  // a block part may end after any group of the tile
+                    if (++cg == gpb && cb < b_end) {
+                        flush();
+                    }
+                }
             }
         }
-        if (it & 1u) {  // both halves of the block are in m
-            m = wave_max(m);
-            if (lane == 0) {
-                out[b_begin + (it >> 1)] = m * out_scale;
+        if constexpr (WR == 1) {
+            // the tile's last fragment was waited for: its buffer is free
+            if (it + 2u < n_tiles) {
+                issue_tile(buf);
             }
-            m = -FLT_MAX;
+        }
+        if constexpr (!SEG) {
+            cg += WR;
+            if (cg == gpb) {
+                flush();
+            }
         }
     }
 }
@@ -424,13 +518,47 @@ __global__ __launch_bounds__(256) void score_fold_kernel(const float *partial, u
 }
 
 size_t score_partial_bytes(uint32_t L, uint32_t Hkv, uint32_t B, uint32_t n_q_tokens, uint32_t g) {
+    // the most any launch shape uses: four partial maxima per row slice and
+    // block (waves times key parts), whatever the block count
     const size_t rows = static_cast<size_t>(n_q_tokens) * g;
-    const size_t slices = (rows + kRowsPerGroup - 1) / kRowsPerGroup * kScoreWaves;
+    const size_t slices = (rows + kSliceRows - 1) / kSliceRows * kMaxRowWaves;
     return sizeof(float) * slices * L * Hkv * B;
 }
 
+using ScoreKernel = void (*)(ScoreParams);
+
+// The kernel of a shape: RT row tiles per wave, WR waves on a key tile, SEG
+// when a block part is not a whole number of tiles, REUSE when several row
+// slices (of four waves then) read the same keys.
+template <int D, int WR, bool SEG, bool REUSE>
+static ScoreKernel score_kernel_of(uint32_t rt) {
+    switch (rt) {
+        case 4: return score_kernel<D, 4, WR, SEG, REUSE>;
+        case 5: return score_kernel<D, 5, WR, SEG, REUSE>;
+        default: return score_kernel<D, 6, WR, SEG, REUSE>;
+    }
+}
+template <int D>
+static ScoreKernel score_kernel_of(uint32_t rt, uint32_t wr, bool seg, bool reuse) {
+    if (wr == 1) {
+        switch (rt) {
+            case 1: return score_kernel<D, 1, 1, false, false>;
+            case 2: return score_kernel<D, 2, 1, false, false>;
+            case 3: return score_kernel<D, 3, 1, false, false>;
+            default: return score_kernel_of<D, 1, false, false>(rt);
+        }
+    }
+    if (wr == 2) {
+        return seg ? score_kernel_of<D, 2, true, false>(rt) : score_kernel_of<D, 2, false, false>(rt);
+    }
+    if (reuse) {
+        return seg ? score_kernel_of<D, 4, true, true>(rt) : score_kernel_of<D, 4, false, true>(rt);
+    }
+    return seg ? score_kernel_of<D, 4, true, false>(rt) : score_kernel_of<D, 4, false, false>(rt);
+}
+
 bool load_score_kernels() {
-    return load_kernel_object(&score_kernel<256>);
+    return load_kernel_object(&score_kernel<256, kMaxRowTiles, kMaxRowWaves, false, false>);
 }
 
 }  // namespace kvmem_hip
@@ -441,8 +569,15 @@ namespace {
 
 // Validates a scorer call and fills its launch shape (everything but the
 // partial-maxima buffer).  Sets *empty when there is nothing to score.
+struct ScoreShape {
+    uint32_t rt = 0;  // row tiles per wave
+    uint32_t wr = 0;  // waves of a workgroup (on one key tile)
+    bool seg = false;
+    uint64_t grid = 0;
+};
+
 int score_setup(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist, const kvmem_hip_score_args *args,
-                ScoreParams &p, uint64_t &grid, bool *empty) {
+                ScoreParams &p, ScoreShape &shape, bool *empty) {
     *empty = false;
     if (!hist || !args || !hist->k || !args->q || !args->scores) {
         return fail(ctx, KVMEM_HIP_ERR_INVALID, "score: null argument");
@@ -492,32 +627,57 @@ int score_setup(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist, const kvmem_h
     p.last_T = hist->last_block_tokens;
     p.g = args->n_head / args->n_head_kv;
     p.R = p.Tq * p.g;
-    p.RG = (p.R + kRowsPerGroup - 1) / kRowsPerGroup;
     p.q_bf16 = args->q_type == KVMEM_TYPE_BF16;
     p.scale = 1.0f / std::sqrt(static_cast<float>(D));
+    // Row slices of at most 24 tiles, equal but for the last; a slice's tiles
+    // go to one wave while they fit its registers, else to two or four waves
+    // that share each key tile.
+    const uint32_t row_tiles = (p.R + 15u) / 16u;
+    p.RG = (row_tiles + kSliceTiles - 1u) / kSliceTiles;
+    const uint32_t slice_tiles = (row_tiles + p.RG - 1u) / p.RG;
+    shape.wr = slice_tiles <= 6u ? 1u : slice_tiles <= 12u ? 2u : 4u;
+    shape.rt = (slice_tiles + shape.wr - 1u) / shape.wr;
+    p.slice_rows = shape.rt * shape.wr * 16u;
     const uint32_t pairs = L * p.Hkv;
-    // two workgroups per CU hold their LDS double buffers; eight per CU
-    // over the launch keep every XCD busy to the end
-    const uint32_t target = 2048;
-    const uint32_t per_chunk_target = std::max<uint32_t>(1, target / std::max<uint32_t>(1, pairs * p.RG));
-    p.n_chunks = std::min(B, per_chunk_target);
-    p.blocks_per_chunk = (B + p.n_chunks - 1) / p.n_chunks;
+    // Few blocks: their keys are split over up to four waves' workgroups
+    const uint32_t groups = (p.T + 15u) / 16u;  // 16-key groups of a block
+    p.KS = 1;
+    while (p.KS * shape.wr < kMaxRowWaves && groups % (2u * p.KS) == 0 &&
+           static_cast<uint64_t>(pairs) * p.RG * B * p.KS * shape.wr < kSplitWaves) {
+        p.KS *= 2u;
+    }
+    p.gpb = groups / p.KS;
+    shape.seg = shape.wr > 1u && p.gpb % shape.wr != 0;
+    // Workgroups of a launch: the chip full once, or two or four times where
+    // that leaves them chunks of 32 or 64 blocks (of 128 keys).  More rounds
+    // even out the end of the launch (16 x 2048 blocks, 64-token query: 2.427
+    // ms with four, 2.447 with one); every workgroup loads and converts its
+    // query rows first, which short chunks do not repay (16 x 128 blocks:
+    // 181 us with four rounds, 163 with one).
+    const uint32_t n_sub = p.RG * p.KS;
+    // (D = 256: 16 KiB of key tiles per wave hold two waves per SIMD)
+    const uint32_t full =
+        1024u * (D == 256 ? 2u : static_cast<uint32_t>(score_occupancy(128, static_cast<int>(shape.rt))));
+    const uint64_t waves = static_cast<uint64_t>(pairs) * n_sub * shape.wr;  // per chunk
+    for (uint32_t rounds = 4; rounds > 0; rounds /= 2u) {
+        p.n_chunks = static_cast<uint32_t>(std::min<uint64_t>(B, std::max<uint64_t>(1, full * rounds / waves)));
+        p.blocks_per_chunk = (B + p.n_chunks - 1) / p.n_chunks;
+        if (static_cast<uint64_t>(p.blocks_per_chunk) * p.T >= 2048u * rounds) {
+            break;
+        }
+    }
     if (p.RG > 1) {
         // Several row slices read the same key tiles.  Their workgroups are
-        // consecutive on one XCD, and short chunks keep them close enough
-        // together for each tile to come from that XCD's L2.  At 16 x 8192
-        // blocks with a 512-token query (8 slices), 16 blocks per chunk cut
-        // HBM reads from 5.6 to 1.9 times the key bytes and the call by
-        // 5.7 %.  Shorter chunks lose more in workgroup start-up (query
-        // rows loaded and converted) than they gain.  4 slices do best with
-        // 64 blocks, 2 with 32.
-        const uint32_t most = p.RG >= 8 ? 16u : (p.RG >= 4 ? 64u : 32u);
-        p.blocks_per_chunk = std::min(p.blocks_per_chunk, most);
+        // consecutive on one XCD, and chunks of at most 64 blocks keep them
+        // close enough together for a tile to come from that XCD's L2 (16 x
+        // 8192 blocks, 512-token query: 65.3 ms; 67.6 with 16 blocks per
+        // chunk, 65.7 with 256).
+        p.blocks_per_chunk = std::min(p.blocks_per_chunk, 64u);
     }
     p.n_chunks = (B + p.blocks_per_chunk - 1) / p.blocks_per_chunk;
     p.xcd_major = (pairs % 8u) == 0;
-    grid = static_cast<uint64_t>(pairs) * p.RG * p.n_chunks;
-    if (grid > 0x7fffffffu) {
+    shape.grid = static_cast<uint64_t>(pairs) * n_sub * p.n_chunks;
+    if (shape.grid > 0x7fffffffu) {
         return fail(ctx, KVMEM_HIP_ERR_INVALID, "score: problem too large for one launch");
     }
     return KVMEM_HIP_OK;
@@ -527,18 +687,17 @@ int score_setup(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist, const kvmem_h
 // per-slice maxima, `layers` the per-layer scores.  `timed` brackets the
 // scorer with the profiling events of kPerfScore.
 int score_launch(kvmem_hip_ctx *ctx, const kvmem_hip_score_args *args, const ScoreParams &p,
-                 uint64_t grid, float *layers, bool timed) {
+                 const ScoreShape &shape, float *layers, bool timed) {
     if (injected_fail(ctx, KVMEM_HIP_FAIL_LAUNCH, "score kernel launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
     if (timed) {
         (void) perf_attach(ctx, kPerfScore);  // the scorer's events ride on its launch
     }
-    if (args->head_dim == 256) {
-        ctx_launch(ctx, score_kernel<256>, dim3(static_cast<uint32_t>(grid)), dim3(kScoreThreads), 0, p);
-    } else {
-        ctx_launch(ctx, score_kernel<128>, dim3(static_cast<uint32_t>(grid)), dim3(kScoreThreads), 0, p);
-    }
+    ctx_launch(ctx,
+               args->head_dim == 256 ? score_kernel_of<256>(shape.rt, shape.wr, shape.seg, p.RG > 1)
+                                     : score_kernel_of<128>(shape.rt, shape.wr, shape.seg, p.RG > 1),
+               dim3(static_cast<uint32_t>(shape.grid)), dim3(shape.wr * 64u), 0, p);
     const bool launched = hip_ok(ctx, hipGetLastError(), "score kernel launch");
     if (timed) {
         perf_detach(ctx, kPerfScore, launched);
@@ -549,7 +708,7 @@ int score_launch(kvmem_hip_ctx *ctx, const kvmem_hip_score_args *args, const Sco
     // the fold is not bracketed: a timing event costs the stream a few
     // microseconds, as much as the fold itself
     score_fold_kernel<<<(p.B + kFoldBlocks - 1) / kFoldBlocks, 256, 0, ctx->stream>>>(
-        p.partial, p.RG * kScoreWaves, p.L, p.Hkv, p.B, layers, args->layer_reduce, args->scores);
+        p.partial, p.RG * p.KS * shape.wr, p.L, p.Hkv, p.B, layers, args->layer_reduce, args->scores);
     if (!hip_ok(ctx, hipGetLastError(), "score fold launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
@@ -619,9 +778,9 @@ extern "C" int kvmem_hip_score(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist
         return KVMEM_HIP_ERR_INVALID;
     }
     ScoreParams p;
-    uint64_t grid = 0;
+    ScoreShape shape;
     bool empty = false;
-    int st = score_setup(ctx, hist, args, p, grid, &empty);
+    int st = score_setup(ctx, hist, args, p, shape, &empty);
     if (st != KVMEM_HIP_OK || empty) {
         return st;
     }
@@ -639,7 +798,7 @@ extern "C" int kvmem_hip_score(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist
         }
         layers = static_cast<float *>(ctx->score_layers.ptr);
     }
-    return score_launch(ctx, args, p, grid, layers, true);
+    return score_launch(ctx, args, p, shape, layers, true);
 }
 
 extern "C" int kvmem_hip_score_noalloc(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist,
@@ -648,9 +807,9 @@ extern "C" int kvmem_hip_score_noalloc(kvmem_hip_ctx *ctx, const kvmem_hip_histo
         return KVMEM_HIP_ERR_INVALID;
     }
     ScoreParams p;
-    uint64_t grid = 0;
+    ScoreShape shape;
     bool empty = false;
-    int st = score_setup(ctx, hist, args, p, grid, &empty);
+    int st = score_setup(ctx, hist, args, p, shape, &empty);
     if (st != KVMEM_HIP_OK || empty) {
         return st;
     }
@@ -695,7 +854,7 @@ extern "C" int kvmem_hip_score_noalloc(kvmem_hip_ctx *ctx, const kvmem_hip_histo
     uint8_t *base = static_cast<uint8_t *>(ctx->noalloc_scratch);
     p.partial = reinterpret_cast<float *>(base);
     float *layers = args->layer_scores ? args->layer_scores : reinterpret_cast<float *>(base + layer_off);
-    st = score_launch(ctx, args, p, grid, layers, false);
+    st = score_launch(ctx, args, p, shape, layers, false);
     if (st != KVMEM_HIP_OK) {
         // a launch that failed after the scorer kernel was queued leaves that
         // kernel on the array with no owner record: let it drain first (a

@@ -200,3 +200,53 @@ def test_score_multi_slice_short_chunks(ctx, oracle, Tq):
     assert_close(ls[:, ids], want, "layer scores")
     del k
     torch.cuda.empty_cache()
+
+
+# (head_dim, query heads per KV head, query tokens, block tokens, blocks, last block's tokens):
+# row tiles per wave 1..6 on one, two and four waves, several slices, blocks
+# shorter than a key tile or no multiple of 16, key parts and ragged ends
+SHAPES = [(256, 1, 16, 128, 700, 1), (256, 3, 10, 128, 5, 17), (256, 6, 8, 128, 40, 0), (256, 4, 16, 64, 9, 33),
+          (256, 5, 16, 32, 300, 31), (256, 6, 16, 128, 9, 128), (256, 7, 16, 48, 11, 40), (256, 10, 13, 32, 21, 2),
+          (256, 6, 32, 128, 6, 100), (256, 13, 16, 16, 30, 5), (256, 6, 53, 128, 7, 64), (256, 6, 64, 32, 17, 30),
+          (256, 6, 67, 64, 12, 50), (256, 8, 100, 128, 90, 0), (128, 1, 5, 128, 600, 3), (128, 4, 8, 100, 9, 99),
+          (128, 4, 10, 128, 3, 0), (128, 4, 14, 16, 50, 15), (128, 4, 20, 7, 80, 6), (128, 4, 24, 64, 70, 1),
+          (128, 4, 40, 32, 33, 16), (128, 4, 48, 128, 5, 77), (128, 8, 29, 80, 10, 0), (128, 8, 40, 128, 8, 9),
+          (128, 4, 96, 112, 11, 100), (128, 8, 61, 1, 200, 0),
+          (256, 6, 42, 128, 8, 0), (256, 6, 100, 16, 40, 9), (256, 6, 64, 128, 10, 90), (128, 4, 28, 128, 9, 1),
+          (128, 4, 28, 16, 31, 7), (128, 4, 110, 128, 12, 3)]
+
+
+@pytest.mark.parametrize("D,g,Tq,T,B,last_T", SHAPES)
+def test_score_tile_edges(ctx, D, g, Tq, T, B, last_T):
+    """In every (layer, block) one key, at a place of its own, is four times
+    one query row: its product, a sum of positive terms, is the block's score.
+    Against 64 bits, the 32-bit sum of D products is within D * 2^-24 of it.
+    Rows of the last block past its tokens hold keys that would win."""
+    announce(f"scorer tile edges: D={D} g={g} Tq={Tq} T={T} B={B} last_T={last_T}")
+    L, Hkv = 2, 2
+    Hq = g * Hkv
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(D + 7 * g + 11 * Tq + T)
+    q = torch.randn((L, Tq, Hq, D), generator=gen, device="cuda").half()
+    k = torch.randn((L, B, T, Hkv, D), generator=gen, device="cuda").mul_(0.1).half()
+    nt = last_T or T
+    rng = np.random.default_rng(T * B + Tq)
+    for l in range(L):
+        for b in range(B):
+            j, h = rng.integers(nt if b == B - 1 else T), rng.integers(Hkv)
+            t, hq = rng.integers(Tq), h * g + rng.integers(g)
+            k[l, b, int(j), int(h)] = 4 * q[l, int(t), int(hq)]
+        if nt < T:
+            k[l, B - 1, nt:] = 40 * q[l, 0, 0]
+    s, ls = run_score(ctx, k, q, kv.TYPE_F16, Hq, Hkv, D, last_T)
+    want = torch.full((L, B), -float("inf"), dtype=torch.float64, device="cuda")
+    for l in range(L):
+        for h in range(Hkv):
+            x = k[l, :, :, h].reshape(-1, D).double() @ q[l, :, h * g:(h + 1) * g].reshape(-1, D).double().T
+            x = x.amax(dim=1).view(B, T)
+            x[B - 1, nt:] = -float("inf")
+            want[l] = torch.maximum(want[l], x.amax(dim=1) / D ** 0.5)
+    want = want.cpu().numpy()
+    tol = (D + 4) * 2.0 ** -24
+    assert np.all(np.abs(ls - want) <= tol * np.abs(want))
+    assert np.all(np.abs(s - want.mean(0)) <= 2 * tol * np.abs(want.mean(0)))
