@@ -4,7 +4,7 @@
 //
 // Producer: k_sum[l][b][e] = fp32 sum of the block's F16 keys in token
 // order, mean_tokens[l][b] = tokens summed (RawKvStore::capture_mean_f16,
-// kvmem/src/host/raw_kv_store.cpp:184-202).  A thread owns 8 consecutive
+// kvmem/src/host/raw_kv_store.cpp:184-202).  A thread owns four consecutive
 // channels and adds token after token, so every channel's sum is the same
 // sequence of IEEE additions as the reference's: bit-identical.
 //
@@ -27,44 +27,130 @@
 
 namespace kvmem_hip {
 
-// grid: (items * L) workgroups of E/8 threads; item i = block_ids[i].  The
+// acc + the f16 value in the low or high half of w, rounded once: the f16
+// operand is widened exactly, so fma(h, 1, acc) is the IEEE sum.
+__device__ inline float add_lo(float acc, uint32_t w) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(acc));
+    return r;
+}
+__device__ inline float add_hi(float acc, uint32_t w) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(acc));
+    return r;
+}
+
+// grid: (items * L) workgroups of E/CH threads; item i = block_ids[i].  The
 // keys of (block b, layer l) are T rows of E halves at k + b*block_stride +
 // l*layer_stride: a device history [L][cap][T][E] or the K rows of a
-// block-major pinned host history.
-__global__ __launch_bounds__(256) void meank_sum_kernel(const uint8_t *k, uint64_t block_stride,
-                                                        uint64_t layer_stride, const uint32_t *items,
-                                                        uint32_t L, uint32_t cap, uint32_t T,
-                                                        uint32_t E, uint32_t last_block,
-                                                        uint32_t last_tokens, float *k_sum,
-                                                        uint32_t *mean_tokens) {
+// block-major pinned host history.  A thread owns CH consecutive channels
+// and adds its rows in token order; the rows of the next batch are loaded
+// before the last batch is added, so a wave waits for memory once per batch
+// and the additions (one v_fma_mix per element) run under the loads.  16
+// blocks x 16 layers of 1024 channels (67 MB of keys): 10.6 us; 44.4 when a
+// wave waited for every row.  All of 512 blocks: 361 us = 6.0 TB/s (421).
+// Four channels per thread: eight (half the waves, each with twice the
+// additions in its chain) take 11.05 and 365 us.
+constexpr uint32_t kSumBatch = 16;
+constexpr int kSumChannels = 4;
+
+template <int CH>
+__global__ __launch_bounds__(2048 / CH) void meank_sum_kernel(const uint8_t *k, uint64_t block_stride,
+                                                              uint64_t layer_stride, const uint8_t *ids_dev,
+                                                              ArgTables ids_args, uint32_t L, uint32_t cap,
+                                                              uint32_t T, uint32_t E, uint32_t last_block,
+                                                              uint32_t last_tokens, float *k_sum,
+                                                              uint32_t *mean_tokens) {
+    typedef uint32_t word_t __attribute__((ext_vector_type(CH / 2)));
+    typedef float sums_t __attribute__((ext_vector_type(4)));
     const uint32_t job = blockIdx.x;
     const uint32_t item = job / L;
     const uint32_t l = job - item * L;
-    const uint32_t b = items[item];
-    const uint32_t e0 = threadIdx.x * 8u;
+    const uint32_t b = tab_read<uint32_t>(ids_dev, ids_args, 4u * item);
+    const uint32_t e0 = threadIdx.x * CH;
     if (e0 >= E) {
         return;
     }
     const uint32_t nt = (b == last_block && last_tokens != 0) ? last_tokens : T;
     const uint8_t *base = k + b * block_stride + l * layer_stride + e0 * 2u;
-    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t t = 0; t < nt; ++t) {
-        const uint4 raw = *reinterpret_cast<const uint4 *>(base + static_cast<uint64_t>(t) * E * 2u);
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    const uint32_t row = E * 2u;
+    auto load = [&](uint32_t t) {
+        return __builtin_nontemporal_load(
+            reinterpret_cast<const word_t *>(base + static_cast<uint64_t>(t) * row));
+    };
+    float s[CH];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            s[2 * i] += static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w[i] & 0xffffu)));
-            s[2 * i + 1] += static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w[i] >> 16)));
+    for (int i = 0; i < CH; ++i) {
+        s[i] = 0.0f;
+    }
+    auto add = [&](word_t w) {
+#pragma unroll
+        for (int i = 0; i < CH / 2; ++i) {
+            s[2 * i] = add_lo(s[2 * i], w[i]);
+            s[2 * i + 1] = add_hi(s[2 * i + 1], w[i]);
+        }
+    };
+    word_t cur[kSumBatch];
+    uint32_t t = 0;
+    if (nt >= kSumBatch) {
+#pragma unroll
+        for (uint32_t j = 0; j < kSumBatch; ++j) {
+            cur[j] = load(j);
+        }
+        for (; t + 2u * kSumBatch <= nt; t += kSumBatch) {
+            word_t next[kSumBatch];
+#pragma unroll
+            for (uint32_t j = 0; j < kSumBatch; ++j) {
+                next[j] = load(t + kSumBatch + j);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kSumBatch; ++j) {
+                add(cur[j]);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kSumBatch; ++j) {
+                cur[j] = next[j];
+            }
+        }
+    }
+    // the last full batch, with the rows past it already on their way
+    const uint32_t tail0 = nt >= kSumBatch ? t + kSumBatch : 0u;
+    word_t rest[kSumBatch];
+#pragma unroll
+    for (uint32_t j = 0; j < kSumBatch; ++j) {
+        rest[j] = 0;
+        if (tail0 + j < nt) {
+            rest[j] = load(tail0 + j);
+        }
+    }
+    if (nt >= kSumBatch) {
+#pragma unroll
+        for (uint32_t j = 0; j < kSumBatch; ++j) {
+            add(cur[j]);
+        }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kSumBatch; ++j) {
+        if (tail0 + j < nt) {
+            add(rest[j]);
         }
     }
     float *out = k_sum + (static_cast<uint64_t>(l) * cap + b) * E + e0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        out[i] = s[i];
+    for (int i = 0; i < CH; i += 4) {
+        *reinterpret_cast<sums_t *>(out + i) = sums_t{s[i], s[i + 1], s[i + 2], s[i + 3]};
     }
     if (threadIdx.x == 0) {
         mean_tokens[static_cast<uint64_t>(l) * cap + b] = nt;
     }
+}
+
+static void launch_meank_sum(hipStream_t stream, uint32_t jobs, const uint8_t *k, uint64_t block_stride,
+                             uint64_t layer_stride, const LaunchTables &ids, uint32_t L, uint32_t cap, uint32_t T,
+                             uint32_t E, uint32_t last_block, uint32_t last_tokens, float *k_sum,
+                             uint32_t *mean_tokens) {
+    meank_sum_kernel<kSumChannels><<<jobs, E / kSumChannels, 0, stream>>>(
+        k, block_stride, layer_stride, ids.dev, ids.args, L, cap, T, E, last_block, last_tokens, k_sum, mean_tokens);
 }
 
 // Query-sum producer: one thread per (layer, channel) adds the listed
@@ -107,28 +193,99 @@ __global__ __launch_bounds__(256) void q_accumulate_kernel(const QT *q, const ui
     *dst = acc;
 }
 
-// Decode running sum: one thread per channel adds the kept tokens' values
-// in token order (strided K view of type KT).
-template <typename KT>
-__global__ __launch_bounds__(256) void meank_add_kernel(const uint8_t *k, uint32_t n_embd,
-                                                        uint32_t head_dim, uint64_t nb0, uint64_t nb1,
-                                                        uint64_t nb2, uint32_t tok0, uint32_t n_keep,
-                                                        int reset, float *acc, uint32_t *count) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e == 0 && count) {
+// Decode running sum: one lane per channel adds the kept tokens' values in
+// token order (strided K view of type KT).  A call has few channels (1024 in
+// 16 waves' worth) and a chain of additions, so it is latency-bound: the
+// WAVES waves of a workgroup (64 channels) each load a run of 32 tokens at
+// once, and the first wave adds all of them in order, its own from registers
+// and the others' from LDS.  Up to 32 tokens take one wave.  128 tokens x 1024
+// f32 channels: 4.4 us; 52.5 with one token in flight at a time.
+constexpr uint32_t kAddRun = 32;
+
+template <typename KT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void meank_add_kernel(const uint8_t *k, uint32_t n_embd,
+                                                               uint32_t head_dim, uint64_t nb0, uint64_t nb1,
+                                                               uint64_t nb2, uint32_t tok0, uint32_t n_keep,
+                                                               int reset, float *acc, uint32_t *count) {
+    __shared__ float rows[WAVES > 1 ? (WAVES - 1) * kAddRun : 1][64];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t e = blockIdx.x * 64u + lane;
+    const bool live = e < n_embd;
+    if (e == 0 && wave == 0 && count) {
         *count = (reset ? 0u : *count) + n_keep;
     }
-    if (e >= n_embd) {
-        return;
-    }
-    const uint32_t head = e / head_dim;
-    const uint32_t dim = e - head * head_dim;
+    const uint32_t ch = live ? e : 0u;  // (in bounds; not stored)
+    const uint32_t head = ch / head_dim;
+    const uint32_t dim = ch - head * head_dim;
     const uint8_t *base = k + static_cast<uint64_t>(head) * nb1 + static_cast<uint64_t>(dim) * nb0;
-    float s = reset ? 0.0f : acc[e];
-    for (uint32_t t = 0; t < n_keep; ++t) {
-        s += static_cast<float>(*reinterpret_cast<const KT *>(base + static_cast<uint64_t>(tok0 + t) * nb2));
+    float s = (reset || wave != 0) ? 0.0f : acc[ch];
+    for (uint32_t t0 = 0; t0 < n_keep; t0 += WAVES * kAddRun) {
+        const uint32_t mine = t0 + wave * kAddRun;
+        float v[kAddRun];
+#pragma unroll
+        for (uint32_t j = 0; j < kAddRun; ++j) {
+            v[j] = 0.0f;
+            if (mine + j < n_keep) {
+                v[j] = static_cast<float>(
+                    *reinterpret_cast<const KT *>(base + static_cast<uint64_t>(tok0 + mine + j) * nb2));
+            }
+        }
+        if (wave == 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < kAddRun; ++j) {
+                if (mine + j < n_keep) {
+                    s += v[j];
+                }
+            }
+        }
+        if constexpr (WAVES > 1) {
+            if (wave != 0) {
+#pragma unroll
+                for (uint32_t j = 0; j < kAddRun; ++j) {
+                    rows[(wave - 1u) * kAddRun + j][lane] = v[j];
+                }
+            }
+            __syncthreads();
+            if (wave == 0) {
+                const uint32_t left = n_keep - min(n_keep, t0 + kAddRun);
+                const uint32_t n = min(left, (WAVES - 1u) * kAddRun);
+                uint32_t j = 0;
+                for (; j + 16u <= n; j += 16u) {
+                    float x[16];
+#pragma unroll
+                    for (uint32_t i = 0; i < 16u; ++i) {
+                        x[i] = rows[j + i][lane];
+                    }
+#pragma unroll
+                    for (uint32_t i = 0; i < 16u; ++i) {
+                        s += x[i];
+                    }
+                }
+                for (; j < n; ++j) {
+                    s += rows[j][lane];
+                }
+            }
+            __syncthreads();  // the rows are read before the next run overwrites them
+        }
     }
-    acc[e] = s;
+    if (live && wave == 0) {
+        acc[e] = s;
+    }
+}
+
+template <typename KT>
+static void launch_meank_add(hipStream_t stream, const uint8_t *k, uint32_t n_embd, uint32_t head_dim, size_t nb0,
+                             size_t nb1, size_t nb2, uint32_t tok0, uint32_t n_keep, int reset, float *acc,
+                             uint32_t *count) {
+    const uint32_t grid = (n_embd + 63u) / 64u;
+    if (n_keep <= kAddRun) {
+        meank_add_kernel<KT, 1><<<grid, 64, 0, stream>>>(k, n_embd, head_dim, nb0, nb1, nb2, tok0, n_keep, reset,
+                                                         acc, count);
+    } else {
+        meank_add_kernel<KT, 4><<<grid, 256, 0, stream>>>(k, n_embd, head_dim, nb0, nb1, nb2, tok0, n_keep, reset,
+                                                          acc, count);
+    }
 }
 
 // Per-layer 1 / (query rows x group size), 0 for a layer without query
@@ -369,17 +526,17 @@ int kvmem_hip_meank_sums(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist,
         return fail(ctx, KVMEM_HIP_ERR_INVALID, "meank_sums: too many blocks in one call");
     }
     (void) hipSetDevice(ctx->device);
-    const void *items = upload(ctx, block_ids, sizeof(uint32_t) * n, "meank_sums ids");
-    if (!items) {
+    LaunchTables ids;  // in the kernel arguments up to 768 blocks
+    if (!stage_tables(ctx, block_ids, sizeof(uint32_t) * n, ids, "meank_sums ids")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
     if (injected_fail(ctx, KVMEM_HIP_FAIL_LAUNCH, "meank_sums launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
     const uint64_t block_stride = static_cast<uint64_t>(hist->block_tokens) * E * 2u;
-    meank_sum_kernel<<<static_cast<uint32_t>(jobs), E / 8, 0, ctx->stream>>>(
-        static_cast<const uint8_t *>(hist->k), block_stride, block_stride * cap,
-        static_cast<const uint32_t *>(items), hist->n_layers, cap, hist->block_tokens, E,
+    launch_meank_sum(
+        ctx->stream, static_cast<uint32_t>(jobs), static_cast<const uint8_t *>(hist->k), block_stride,
+        block_stride * cap, ids, hist->n_layers, cap, hist->block_tokens, E,
         hist->n_blocks - 1, hist->last_block_tokens, k_sum, mean_tokens);
     return hip_ok(ctx, hipGetLastError(), "meank_sums launch") ? KVMEM_HIP_OK : KVMEM_HIP_ERR_RUNTIME;
 }
@@ -423,15 +580,15 @@ int kvmem_hip_meank_sums_host(kvmem_hip_ctx *ctx, const kvmem_hip_host_history *
         return fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED,
                     "meank_sums_host: the history must lie inside one pinned host allocation");
     }
-    const void *items = upload(ctx, block_ids, sizeof(uint32_t) * n, "meank_sums_host ids");
-    if (!items) {
+    LaunchTables ids;
+    if (!stage_tables(ctx, block_ids, sizeof(uint32_t) * n, ids, "meank_sums_host ids")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
     if (injected_fail(ctx, KVMEM_HIP_FAIL_LAUNCH, "meank_sums_host launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
-    meank_sum_kernel<<<static_cast<uint32_t>(jobs), E / 8, 0, ctx->stream>>>(
-        view, span, layer_bytes, static_cast<const uint32_t *>(items), hist->n_layers, cap, T, E,
+    launch_meank_sum(
+        ctx->stream, static_cast<uint32_t>(jobs), view, span, layer_bytes, ids, hist->n_layers, cap, T, E,
         hist->n_blocks - 1, hist->last_block_tokens, k_sum, mean_tokens);
     if (!hip_ok(ctx, hipGetLastError(), "meank_sums_host launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
@@ -465,17 +622,14 @@ int kvmem_hip_meank_add(kvmem_hip_ctx *ctx, const void *k, int32_t k_type, uint3
         return KVMEM_HIP_OK;
     }
     (void) hipSetDevice(ctx->device);
-    const uint32_t grid = (n_embd + 255) / 256;
     const uint8_t *kb = static_cast<const uint8_t *>(k);
     if (k_type == KVMEM_TYPE_F32) {
-        meank_add_kernel<float><<<grid, 256, 0, ctx->stream>>>(kb, n_embd, head_dim, nb0, nb1, nb2, tok0,
-                                                              n_keep, reset, acc, count);
+        launch_meank_add<float>(ctx->stream, kb, n_embd, head_dim, nb0, nb1, nb2, tok0, n_keep, reset, acc, count);
     } else if (k_type == KVMEM_TYPE_F16) {
-        meank_add_kernel<_Float16><<<grid, 256, 0, ctx->stream>>>(kb, n_embd, head_dim, nb0, nb1, nb2, tok0,
-                                                                 n_keep, reset, acc, count);
+        launch_meank_add<_Float16>(ctx->stream, kb, n_embd, head_dim, nb0, nb1, nb2, tok0, n_keep, reset, acc,
+                                   count);
     } else {
-        meank_add_kernel<__bf16><<<grid, 256, 0, ctx->stream>>>(kb, n_embd, head_dim, nb0, nb1, nb2, tok0,
-                                                               n_keep, reset, acc, count);
+        launch_meank_add<__bf16>(ctx->stream, kb, n_embd, head_dim, nb0, nb1, nb2, tok0, n_keep, reset, acc, count);
     }
     return hip_ok(ctx, hipGetLastError(), "meank_add launch") ? KVMEM_HIP_OK : KVMEM_HIP_ERR_RUNTIME;
 }

@@ -362,3 +362,67 @@ def test_engine_host_only_history_meank(oracle):
                 e2.set_host_history(hb.data_ptr(), cap)
                 e2.append_tokens(nb * T)
                 e2.preview(qd.data_ptr(), Tq)
+
+
+def ordered_sum(rows: np.ndarray) -> np.ndarray:
+    """float32 additions row after row, from zero."""
+    s = np.zeros(rows.shape[1:], np.float32)
+    for r in rows.astype(np.float32):
+        s = s + r
+    return s
+
+
+@pytest.mark.parametrize("n_ids", [1, 6, 800])   # 800 ids do not fit the kernel arguments
+@pytest.mark.parametrize("Tb,last,E_", [(1, 0, 8), (15, 3, 64), (16, 0, 24), (17, 16, 1000), (31, 1, 2048),
+                                        (32, 31, 512), (33, 32, 40), (48, 47, 256), (128, 127, 1024)])
+def test_meank_sums_batch_edges(ctx, n_ids, Tb, last, E_):
+    """Block lengths around the kernel's batches of 16 rows, row widths from 8
+    to 2048 channels, subnormal, signed zero and infinite keys."""
+    announce(f"sums: {Tb}-token blocks (last {last}) of {E_} channels, {n_ids} ids")
+    if n_ids == 800 and E_ > 256:
+        n_ids = 769
+    nb, L_ = (n_ids if n_ids < 800 else 800), 2
+    g = torch.Generator(device="cuda").manual_seed(Tb * E_)
+    k = (torch.randn((L_, nb, Tb, E_), generator=g, device="cuda") * 50).half()
+    k[..., 0] = -0.0
+    k[..., 1] = 6e-8                                  # the smallest f16 subnormal
+    k[0, 0, 0, 2] = float("inf")
+    ks = torch.full((L_, nb, E_), float("nan"), dtype=torch.float32, device="cuda")
+    mt = torch.zeros((L_, nb), dtype=torch.int32, device="cuda")
+    hist = ctx.make_history(k.data_ptr(), None, L_, nb, Tb, E_, 0, last)
+    torch.cuda.synchronize()
+    ids = np.random.default_rng(3).permutation(nb)[:n_ids].tolist()
+    ctx.meank_sums(hist, ids, ks.data_ptr(), mt.data_ptr())
+    ctx.sync()
+    kn, got, n_tok = k.cpu().numpy(), ks.cpu().numpy(), mt.cpu().numpy()
+    full = ordered_sum(kn.transpose(2, 0, 1, 3))
+    if last:
+        full[:, nb - 1] = ordered_sum(kn[:, nb - 1, :last].transpose(1, 0, 2))
+    assert np.array_equal(got.view(np.uint32), full.view(np.uint32))
+    assert np.all(n_tok[:, :nb - 1] == Tb) and np.all(n_tok[:, nb - 1] == (last or Tb))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n,heads,Dh", [(1, 4, 256), (31, 3, 8), (32, 1, 64), (33, 2, 128), (64, 5, 40),
+                                        (127, 1, 1), (128, 4, 256), (129, 8, 128), (300, 3, 72)])
+def test_meank_add_run_edges(ctx, dtype, n, heads, Dh):
+    """Token counts around the kernel's runs of 32 and 128, channel counts
+    that do not fill a wave, from a first token past 0; continued by the same
+    rows."""
+    announce(f"running key sum: {n} tokens x {heads} heads x {Dh}, {dtype}")
+    tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    code = {"f32": kv.TYPE_F32, "f16": kv.TYPE_F16, "bf16": kv.TYPE_BF16}[dtype]
+    g = torch.Generator(device="cuda").manual_seed(n + Dh)
+    full = (torch.randn((n + 5, heads, Dh + 3), generator=g, device="cuda") * 1000).to(tdt)
+    esz, ne = full.element_size(), heads * Dh
+    acc = torch.full((ne + 64,), float("nan"), dtype=torch.float32, device="cuda")
+    cnt = torch.full((2,), 7, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    strides = (esz, (Dh + 3) * esz, heads * (Dh + 3) * esz)
+    for reset in (True, False):
+        ctx.meank_add(full.data_ptr(), code, ne, Dh, *strides, 5, n, acc.data_ptr(), cnt.data_ptr(), reset=reset)
+    ctx.sync()
+    rows = full[5:, :, :Dh].float().cpu().numpy().reshape(n, ne)
+    got = acc.cpu().numpy()
+    assert np.array_equal(got[:ne].view(np.uint32), ordered_sum(np.concatenate([rows, rows])).view(np.uint32))
+    assert np.isnan(got[ne:]).all() and cnt.tolist() == [2 * n, 7]
