@@ -374,3 +374,59 @@ def test_set_query_then_unfrozen_rows_add_on(oracle):
         eng.reset_query()                               # the state and the rows go
         with pytest.raises(kv.KvMemError):
             eng.get_query()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("heads,hd,pad,shift,n,first", [
+    (1, 4, 0, 0, 3, 0),          # one unit of a wave-wide access
+    (3, 12, 0, 0, 5, 0),         # rows of 36 elements
+    (24, 256, 0, 0, 7, 0),       # three workgroups per row, contiguous heads
+    (8, 260, 0, 0, 400, 0),      # a row just past a workgroup's 2048 elements
+    (3, 6, 0, 0, 4, 0),          # rows of 18: element by element
+    (4, 64, 8, 0, 6, 0),         # padded heads: element by element
+    (4, 64, 0, 1, 6, 0),         # window rows 4 bytes off a 16-byte boundary
+    (2, 16, 0, 0, 900, 0),       # more pairs than the kernel arguments hold
+    (2, 16, 0, 0, 20, 65530),    # tokens past 16 bits
+])
+def test_window_write_row_forms(dtype, heads, hd, pad, shift, n, first):
+    """Every form of a captured row: widened exactly, nothing else written."""
+    announce(f"q_window_write: {n} rows of {heads} x {hd} (+{pad}), {dtype}, first token {first}")
+    tdt, code = DTYPES[dtype]
+    cap, e = n + 9, heads * hd
+    g = torch.Generator(device="cuda").manual_seed(e + n)
+    q = torch.randn((first + n, heads, hd + pad), generator=g, device="cuda").to(tdt)
+    win = torch.full((shift + cap * e,), -7.0, dtype=torch.float32, device="cuda")
+    rng = np.random.default_rng(n)
+    tokens = first + rng.permutation(n)
+    rows = rng.permutation(cap)[:n]
+    esz = q.element_size()
+    torch.cuda.synchronize()
+    with kv.Context(0) as ctx:
+        ctx.q_window_write(q.data_ptr(), code, heads, hd, esz, (hd + pad) * esz, heads * (hd + pad) * esz,
+                           tokens.tolist(), rows.tolist(), win.data_ptr() + 4 * shift, cap)
+        ctx.sync()
+    want = np.full((cap, e), -7.0, np.float32)
+    want[rows] = q[:, :, :hd].float().cpu().numpy().reshape(first + n, e)[tokens]
+    got = win.cpu().numpy()
+    assert np.array_equal(got[shift:].reshape(cap, e).view(np.uint32), want.view(np.uint32))
+    assert np.all(got[:shift] == -7.0)
+
+
+@pytest.mark.parametrize("e,shift", [(8, 0), (2048, 0), (2056, 0), (6144, 0), (12, 0), (1, 0), (64, 1)])
+def test_window_gather_row_forms(e, shift):
+    """Row widths around the 2048 elements of a workgroup, widths that are no
+    multiple of 8 and an output off a 16-byte boundary, in every type."""
+    announce(f"q_window_gather: rows of {e} elements, output shifted by {shift}")
+    n_layers, cap, rows = 3, 5, [4, 0, 4, 1]
+    win = np.random.default_rng(e).standard_normal((n_layers, cap, e)).astype(np.float32) * 100
+    wd = torch.from_numpy(win).cuda()
+    want = np.ascontiguousarray(win[:, rows])
+    with kv.Context(0) as ctx:
+        for tdt, ty in ((torch.float32, kv.TYPE_F32), (torch.bfloat16, kv.TYPE_BF16), (torch.float16, kv.TYPE_F16)):
+            out = torch.full((shift + want.size + 8,), 3.0, dtype=tdt, device="cuda")
+            torch.cuda.synchronize()
+            ctx.q_window_gather(wd.data_ptr(), n_layers, cap, e, rows, ty, out.data_ptr() + shift * out.element_size())
+            ctx.sync()
+            ref = torch.from_numpy(want).to(tdt).reshape(-1)
+            assert torch.equal(out[shift:shift + want.size].cpu(), ref)
+            assert bool((out[:shift] == 3).all()) and bool((out[shift + want.size:] == 3).all())
