@@ -671,7 +671,7 @@ def run_meank_256k(a, torch, kv, workloads, tensors=None) -> dict:
     return {"metric": "reselect @256K with the mean-K cosine scorer", "unit": "ms/step",
             "value": round(m["ms_step"], 4), "higher_is_better": False, "n_gpus": 1,
             "steps": a.steps, "warmup": a.warmup, "data": "synthetic (seeded N(0,1) keys, bf16 query)",
-            "score_roofline": {"bound": "hbm", "kernel": "meank_cos_kernel<256>",
+            "score_roofline": {"bound": "hbm", "kernel": "meank_score_kernel<256>",
                                "achieved": round(sums_bytes / (m["cos_ms"] * 1e-3) / 1e9, 1),
                                "peak": HBM_PEAK_GBS, "unit": "GB/s", "algorithmic_bytes": sums_bytes,
                                "frac": round(sums_bytes / (m["cos_ms"] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),

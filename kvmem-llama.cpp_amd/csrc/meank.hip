@@ -289,19 +289,23 @@ static void launch_meank_add(hipStream_t stream, const uint8_t *k, uint32_t n_em
 }
 
 // Per-layer 1 / (query rows x group size), 0 for a layer without query
-// rows, carried in the query kernel's arguments (no upload before it).
+// rows, carried in the kernels' arguments (no upload before them).
 constexpr uint32_t kMeankMaxL = 256;
 struct LayerScales {
     float v[kMeankMaxL];
 };
+// The layers with query rows, ascending.
+struct ScoredLayers {
+    uint32_t n;
+    uint32_t l[kMeankMaxL];
+};
 
 // One workgroup per (layer, KV head), one thread per channel: the group's
-// query sum (heads added in group order) scaled by invq, and its squared
-// norm reduced over the channels.  The (layer, 0) workgroups also copy the
-// layer's scale to invq_out in device memory for the kernels after it.
-__global__ __launch_bounds__(256) void meank_query_kernel(const float *q_sum, LayerScales invq,
-                                                          float *invq_out, uint32_t L, uint32_t Hq,
-                                                          uint32_t Hkv, uint32_t D, float *qv, float *nq) {
+// query sum (heads added in group order, their loads issued eight at a time)
+// scaled by invq, and its norm, reduced over the channels.
+__global__ __launch_bounds__(256) void meank_query_kernel(const float *q_sum, LayerScales invq, uint32_t L,
+                                                          uint32_t Hq, uint32_t Hkv, uint32_t D, float *qv,
+                                                          float *nq) {
     __shared__ float part[4];
     const uint32_t i = blockIdx.x;  // l * Hkv + h
     const uint32_t d = threadIdx.x;
@@ -309,14 +313,23 @@ __global__ __launch_bounds__(256) void meank_query_kernel(const float *q_sum, La
     const uint32_t h = i - l * Hkv;
     const uint32_t g = Hq / Hkv;
     const float scale = invq.v[l];  // uniform index: read from the argument bytes
-    if (h == 0 && d == 0) {
-        invq_out[l] = scale;
-    }
     float v = 0.0f;
     if (d < D) {
+        constexpr uint32_t kBatch = 8;
+        const float *src = q_sum + (static_cast<uint64_t>(l) * Hq + h * g) * D + d;
         float acc = 0.0f;
-        for (uint32_t gi = 0; gi < g; ++gi) {
-            acc += q_sum[(static_cast<uint64_t>(l) * Hq + h * g + gi) * D + d];
+        for (uint32_t g0 = 0; g0 < g; g0 += kBatch) {
+            float x[kBatch];
+#pragma unroll
+            for (uint32_t j = 0; j < kBatch; ++j) {
+                x[j] = g0 + j < g ? src[static_cast<uint64_t>(g0 + j) * D] : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kBatch; ++j) {
+                if (g0 + j < g) {
+                    acc += x[j];
+                }
+            }
         }
         v = acc * scale;
         qv[static_cast<uint64_t>(i) * D + d] = v;
@@ -335,7 +348,7 @@ __global__ __launch_bounds__(256) void meank_query_kernel(const float *q_sum, La
         for (uint32_t w = 0; w < (blockDim.x + 63u) / 64u; ++w) {
             t += part[w];
         }
-        nq[i] = t;
+        nq[i] = sqrtf(t);
     }
 }
 
@@ -354,137 +367,189 @@ __device__ inline float row16_sum(float v) {
     return v;
 }
 
-// 16 lanes per (layer, block) item, 16 items per 256-thread workgroup.  A
-// lane holds D/16 channels of each head as float4s.  The key sums of every
-// head (up to kMaxHeads) are loaded before the first head is reduced, so an
-// item waits for memory once; the query vectors (shared by the layer's
-// blocks, cache hits) are loaded per head.
-template <int D>
-__global__ __launch_bounds__(256) void meank_cos_kernel(const float *k_sum, const uint32_t *mean_tokens,
-                                                        const float *qv, const float *nq,
-                                                        const float *invq, uint32_t L, uint32_t B,
-                                                        uint32_t cap, uint32_t Hkv, double *layer_cos) {
+// Cosines and their combination over layers: a workgroup of 8 waves takes
+// groups of 4 blocks, every layer of them.  Wave w scores the scored layers w,
+// w + 8, ..., 16 lanes per block: a lane holds D/16 channels of HS heads as
+// float4s (16 KiB per wave with HS = 4 and D = 256), all loaded before the
+// first is reduced, and the next step's loads are issued as soon as the last
+// head is, before the group's layers meet.  The query vectors come from LDS
+// when every layer's fit there (QLDS: loads return in order, so a query load
+// behind key loads would wait for all of them), else from the caches.  The
+// layers' cosine sums meet in LDS, where one thread per block adds them in
+// layer order (in double): the mean over scored layers of the cosine sum / Hkv,
+// 0 when no layer holds keys of the block.  HBM-bound: every key sum is read
+// once.  16 layers x 2048 blocks of 1024 channels (134 MB): 24.1 us = 5.6 TB/s,
+// where a kernel for the cosines and one for the combination took 34.0 and 5.0
+// with a launch between them.  (Query vectors from the caches: 25.1.)
+// Workgroups beyond two per CU would start late and run alone: 2100 blocks take
+// 58.3 us per preview with 512 workgroups that go on to the next group, 60.7
+// with one workgroup per group.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+constexpr uint32_t kCosBlocks = 4;
+constexpr uint32_t kCosWaves = 8;
+constexpr uint32_t kCosGroups = 512;      // workgroups of a launch, at most: two per CU
+constexpr uint32_t kCosLds = 79 * 1024;   // LDS that leaves room for two workgroups per CU
+extern __shared__ float4 cos_lds[];
+
+// Dynamic LDS: the layers' cosine sums of two groups, then (QLDS) the query
+// vectors and their norms.
+static size_t cos_lds_bytes(uint32_t L, uint32_t Hkv, uint32_t D, bool q_lds) {
+    const size_t term = sizeof(double) * 2u * kCosBlocks * L;
+    return term + (q_lds ? sizeof(float) * static_cast<size_t>(L) * Hkv * (D + 1u) : 0u);
+}
+
+template <int D, int HS, bool QLDS>
+__global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void meank_score_kernel(
+    const float *k_sum, const uint32_t *mean_tokens, const float *qv, const float *nq, ScoredLayers scored, uint32_t L,
+    uint32_t B, uint32_t cap, uint32_t Hkv, float *scores) {
     constexpr int P4 = D / 64;  // float4s per lane per head
-    constexpr int kMaxHeads = 4;  // heads whose key sums are in flight together
-    const uint32_t item = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const uint32_t sub = threadIdx.x & 15u;
-    const bool live = item < L * B;
-    const uint32_t l = live ? item / B : 0u;
-    const uint32_t b = live ? item - l * B : 0u;
-    const float iq = invq[l];
-    const uint32_t mt_raw = mean_tokens[static_cast<uint64_t>(l) * cap + b];
-    const bool scored = live && iq != 0.0f;  // layers without query rows are skipped
-    const uint32_t mt = scored ? mt_raw : 0u;
-    const float inv = mt ? 1.0f / static_cast<float>(mt) : 0.0f;
-    const float4 *ks = reinterpret_cast<const float4 *>(k_sum + (static_cast<uint64_t>(l) * cap + b) * Hkv * D);
-    const float4 *qs = reinterpret_cast<const float4 *>(qv + static_cast<uint64_t>(l) * Hkv * D);
-    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    double layer = 0.0;
-    for (uint32_t h0 = 0; h0 < Hkv; h0 += kMaxHeads) {
-        const uint32_t nh = min(Hkv - h0, static_cast<uint32_t>(kMaxHeads));
-        float4 kc[kMaxHeads][P4];
+    __shared__ uint32_t has_keys[2][kCosWaves][kCosBlocks];
+    double *term = reinterpret_cast<double *>(cos_lds);  // [2][kCosBlocks][L]
+    f32x4_t *q_lds = reinterpret_cast<f32x4_t *>(cos_lds) + kCosBlocks * L;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t sub = lane & 15u;
+    const uint32_t lb = lane >> 4;
+    const uint32_t row4 = Hkv * (D / 4);  // float4s of a key-sum row
+    const uint32_t n_groups = (B + kCosBlocks - 1u) / kCosBlocks;
+
+    // a step: HS heads of one scored layer, loaded together
+    f32x4_t kc[HS][P4];
+    auto block_of = [&](uint32_t g) { return min(g * kCosBlocks + lb, B - 1u); };  // past the end: not stored
+    auto load_step = [&](uint32_t g, uint32_t l, uint32_t h0) {
+        const f32x4_t *row = reinterpret_cast<const f32x4_t *>(k_sum) +
+                             (static_cast<uint64_t>(l) * cap + block_of(g)) * row4 + sub;
 #pragma unroll
-        for (int hh = 0; hh < kMaxHeads; ++hh) {
+        for (int hh = 0; hh < HS; ++hh) {
+            const f32x4_t *src = row + min(h0 + hh, Hkv - 1u) * (D / 4);  // past the last head: it again, not used
 #pragma unroll
             for (int j = 0; j < P4; ++j) {
-                // loaded whatever mt is (every row up to capacity is in bounds),
-                // chosen after: the load need not wait for mean_tokens
-                const float4 kv = static_cast<uint32_t>(hh) < nh ? ks[(h0 + hh) * (D / 4) + j * 16 + sub] : zero;
-                kc[hh][j] = mt ? kv : zero;
+                // whatever the layer's mean_tokens: every row up to capacity is in bounds
+                kc[hh][j] = __builtin_nontemporal_load(src + j * 16);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);  // all of them before the first use
+    };
+    auto load_tokens = [&](uint32_t g, uint32_t l) { return mean_tokens[static_cast<uint64_t>(l) * cap + block_of(g)]; };
+    uint32_t g = blockIdx.x;  // (the grid has at most n_groups workgroups)
+    uint32_t mt = 0;          // tokens of the step's layer in the lane's block
+    if (wave < scored.n) {
+        mt = load_tokens(g, scored.l[wave]);
+        load_step(g, scored.l[wave], 0u);
+    }
+    const float *q_norm = nq;
+    if constexpr (QLDS) {
+        const f32x4_t *src = reinterpret_cast<const f32x4_t *>(qv);
+        for (uint32_t t = threadIdx.x; t < L * row4; t += kCosWaves * 64u) {
+            q_lds[t] = src[t];
+        }
+        float *norms = reinterpret_cast<float *>(q_lds + L * row4);
+        for (uint32_t t = threadIdx.x; t < L * Hkv; t += kCosWaves * 64u) {
+            norms[t] = nq[t];
+        }
+        __syncthreads();
+        q_norm = norms;
+    }
+    uint32_t turn = 0;
+    for (; g < n_groups; g += gridDim.x, turn ^= 1u) {
+        uint32_t has = 0;
+        for (uint32_t i = wave; i < scored.n; i += kCosWaves) {
+            const uint32_t l = scored.l[i];
+            const f32x4_t *qs = (QLDS ? q_lds : reinterpret_cast<const f32x4_t *>(qv)) + l * row4 + sub;
+            const float inv = mt ? 1.0f / static_cast<float>(mt) : 0.0f;
+            double layer = 0.0;
+            for (uint32_t h0 = 0; h0 < Hkv; h0 += HS) {
+                if (h0 != 0) {
+                    load_step(g, l, h0);
+                }
+                if (mt == 0u) {  // no keys: whatever the row holds does not count
 #pragma unroll
-        for (int hh = 0; hh < kMaxHeads; ++hh) {
-            if (static_cast<uint32_t>(hh) >= nh) {
-                break;
-            }
-            const uint32_t h = h0 + hh;
-            float dot = 0.0f, nk = 0.0f;
+                    for (int hh = 0; hh < HS; ++hh) {
 #pragma unroll
-            for (int j = 0; j < P4; ++j) {
-                const float4 qv4 = qs[h * (D / 4) + j * 16 + sub];
-                const float4 qc = scored ? qv4 : zero;
-                const float m[4] = {kc[hh][j].x * inv, kc[hh][j].y * inv, kc[hh][j].z * inv, kc[hh][j].w * inv};
-                const float q[4] = {qc.x, qc.y, qc.z, qc.w};
+                        for (int j = 0; j < P4; ++j) {
+                            kc[hh][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                        }
+                    }
+                }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    dot += q[e] * m[e];
-                    nk += m[e] * m[e];
+                for (int hh = 0; hh < HS; ++hh) {
+                    const uint32_t h = min(h0 + hh, Hkv - 1u);
+                    float dot = 0.0f, nk = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < P4; ++j) {
+                        const f32x4_t q = qs[h * (D / 4) + j * 16];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float m = kc[hh][j][e] * inv;
+                            dot = __builtin_fmaf(q[e], m, dot);
+                            nk = __builtin_fmaf(m, m, nk);
+                        }
+                    }
+                    dot = row16_sum(dot);
+                    nk = row16_sum(nk);
+                    if (h0 + hh < Hkv) {
+                        layer += static_cast<double>(dot / (q_norm[l * Hkv + h] * sqrtf(nk) + 1e-6f));
+                    }
                 }
             }
-            dot = row16_sum(dot);
-            nk = row16_sum(nk);
-            const float nqh = nq[l * Hkv + h];
-            const float c = dot / (sqrtf(scored ? nqh : 0.0f) * sqrtf(nk) + 1e-6f);
-            layer += static_cast<double>(c);
+            has |= mt;
+            // the wave's next step: its next layer, or its first of the next group
+            const bool more = i + kCosWaves < scored.n;
+            const uint32_t gn = more ? g : g + gridDim.x;
+            if (gn < n_groups) {
+                const uint32_t ln = scored.l[more ? i + kCosWaves : wave];
+                mt = load_tokens(gn, ln);
+                load_step(gn, ln, 0u);
+            }
+            if (sub == 0u) {
+                term[(turn * kCosBlocks + lb) * L + i] = layer / static_cast<double>(Hkv);
+            }
         }
-    }
-    if (scored && sub == 0u) {
-        layer_cos[static_cast<uint64_t>(l) * B + b] = layer;
+        if (scored.n != L) {  // the layers without query rows count here too
+            for (uint32_t u = wave; u < L; u += kCosWaves) {
+                has |= load_tokens(g, u);
+            }
+        }
+        if (sub == 0u) {
+            has_keys[turn][wave][lb] = has;
+        }
+        __syncthreads();  // (the next group's terms go to the other half)
+        const uint32_t t = threadIdx.x;
+        const uint32_t b = g * kCosBlocks + t;
+        if (t < kCosBlocks && b < B) {
+            uint32_t any = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < kCosWaves; ++w) {
+                any |= has_keys[turn][w][t];
+            }
+            double acc = 0.0;
+            for (uint32_t u = 0; u < scored.n; ++u) {
+                acc += term[(turn * kCosBlocks + t) * L + u];
+            }
+            scores[b] = static_cast<float>((any && scored.n) ? acc / scored.n : 0.0);
+        }
     }
 }
 
-// A block's score: the mean over scored layers of its layer cosine sum / Hkv
-// (in double, in layer order); 0 when no layer holds keys of the block.
-// Threads take (layer slice, block) pairs so every load is issued at once:
-// the workgroup covers 256 / kCombineLayers blocks, each thread its block's
-// layers l = slice, slice + kCombineLayers, ..., and one thread per block
-// adds the terms from LDS in layer order.
-constexpr uint32_t kCombineLayers = 16;
-constexpr uint32_t kCombineMaxL = 256;  // layers held in LDS per block
+using MeankScoreKernel = void (*)(const float *, const uint32_t *, const float *, const float *, ScoredLayers, uint32_t,
+                                  uint32_t, uint32_t, uint32_t, float *);
 
-__global__ __launch_bounds__(256) void meank_combine_kernel(const double *layer_cos,
-                                                            const uint32_t *mean_tokens,
-                                                            const float *invq, uint32_t L, uint32_t B,
-                                                            uint32_t cap, uint32_t Hkv, float *scores) {
-    constexpr uint32_t kBlocks = 256 / kCombineLayers;
-    __shared__ double term[kBlocks][kCombineMaxL];
-    __shared__ uint32_t any_keys[kBlocks];
-    const uint32_t lb = threadIdx.x / kCombineLayers;  // block within the workgroup
-    const uint32_t slice = threadIdx.x - lb * kCombineLayers;
-    const uint32_t b = blockIdx.x * kBlocks + lb;
-    if (slice == 0) {
-        any_keys[lb] = 0u;
+template <int D>
+static MeankScoreKernel meank_score_of(uint32_t Hkv, bool q_lds) {
+    // steps of four heads, or of two where four would load heads twice
+    if (Hkv % 4u != 0 && (Hkv + 1u) / 2u * 2u < (Hkv + 3u) / 4u * 4u) {
+        return q_lds ? meank_score_kernel<D, 2, true> : meank_score_kernel<D, 2, false>;
     }
-    __syncthreads();
-    if (b < B) {
-        uint32_t has = 0;
-        for (uint32_t l = slice; l < L; l += kCombineLayers) {
-            has |= mean_tokens[static_cast<uint64_t>(l) * cap + b] != 0 ? 1u : 0u;
-            term[lb][l] = invq[l] != 0.0f ? layer_cos[static_cast<uint64_t>(l) * B + b] : 0.0;
-        }
-        if (has) {
-            atomicOr(&any_keys[lb], 1u);
-        }
-    }
-    __syncthreads();
-    if (b >= B || slice != 0) {
-        return;
-    }
-    double acc = 0.0;
-    uint32_t nlay = 0;
-    for (uint32_t l = 0; l < L; ++l) {
-        if (invq[l] != 0.0f) {
-            acc += term[lb][l] / static_cast<double>(Hkv ? Hkv : 1);
-            ++nlay;
-        }
-    }
-    scores[b] = static_cast<float>((any_keys[lb] && nlay) ? acc / nlay : 0.0);
-}
-
-// Per-(layer, block) cosine sums in double, rounded up to 256 bytes so the
-// query vectors after them start aligned.
-static size_t meank_cos_bytes(uint32_t L, uint32_t B) {
-    return (sizeof(double) * static_cast<size_t>(L) * B + 255) & ~static_cast<size_t>(255);
+    return q_lds ? meank_score_kernel<D, 4, true> : meank_score_kernel<D, 4, false>;
 }
 
 size_t meank_scratch_bytes(uint32_t L, uint32_t Hkv, uint32_t B, uint32_t D) {
-    const size_t qv_bytes = sizeof(float) * static_cast<size_t>(L) * Hkv * (D + 1);
-    return meank_cos_bytes(L, B) + qv_bytes + sizeof(float) * static_cast<size_t>(L) + 256;
+    (void) B;  // the query vectors and their norms; no per-block scratch
+    return sizeof(float) * static_cast<size_t>(L) * Hkv * (D + 1);
 }
 
 bool load_meank_kernels() {
-    return load_kernel_object(&meank_cos_kernel<256>);
+    return load_kernel_object(&meank_score_kernel<256, 4, true>);
 }
 
 }  // namespace kvmem_hip
@@ -700,7 +765,6 @@ int kvmem_hip_score_meank(kvmem_hip_ctx *ctx, const kvmem_hip_meank_args *a) {
     if (reinterpret_cast<uintptr_t>(a->k_sum) & 15u) {
         return fail(ctx, KVMEM_HIP_ERR_INVALID, "score_meank: k_sum must be 16-byte aligned");
     }
-    static_assert(kMeankMaxL == kCombineMaxL, "layer bound");
     if (L > kMeankMaxL) {
         return fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED, "score_meank: more than 256 layers");
     }
@@ -711,35 +775,35 @@ int kvmem_hip_score_meank(kvmem_hip_ctx *ctx, const kvmem_hip_meank_args *a) {
     // per-layer 1 / (q_count * g) as the reference computes it in fp32; 0
     // marks a layer without query rows
     LayerScales invq{};
+    ScoredLayers scored{};
     for (uint32_t l = 0; l < L; ++l) {
+        if (a->q_count[l]) {
+            scored.l[scored.n++] = l;
+        }
         invq.v[l] = a->q_count[l] ? 1.0f / static_cast<float>(a->q_count[l] * g) : 0.0f;
     }
     (void) hipSetDevice(ctx->device);
-    // the fp32 query vectors start 256-byte aligned (read as float4)
-    const size_t cos_bytes = meank_cos_bytes(L, B);
     if (!ensure_dev(ctx, ctx->meank_scratch, meank_scratch_bytes(L, a->n_head_kv, B, D),
                     "score_meank scratch")) {
         return KVMEM_HIP_ERR_NOMEM;
     }
-    uint8_t *scratch = static_cast<uint8_t *>(ctx->meank_scratch.ptr);
-    double *layer_cos = reinterpret_cast<double *>(scratch);
-    float *qv = reinterpret_cast<float *>(scratch + cos_bytes);
+    float *qv = static_cast<float *>(ctx->meank_scratch.ptr);  // read as float4
     float *nq = qv + static_cast<size_t>(L) * a->n_head_kv * D;
-    float *invq_dev = nq + static_cast<size_t>(L) * a->n_head_kv;
     if (injected_fail(ctx, KVMEM_HIP_FAIL_LAUNCH, "score_meank launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
     perf_begin(ctx, kPerfScore);
     const uint32_t lh = L * a->n_head_kv;
-    meank_query_kernel<<<lh, D, 0, ctx->stream>>>(a->q_sum, invq, invq_dev, L, a->n_head, a->n_head_kv, D,
-                                                  qv, nq);
-    const uint64_t items = static_cast<uint64_t>(L) * B;  // 16 lanes each
-    const uint32_t grid = static_cast<uint32_t>((items * 16 + 255) / 256);
+    meank_query_kernel<<<lh, D, 0, ctx->stream>>>(a->q_sum, invq, L, a->n_head, a->n_head_kv, D, qv, nq);
+    const uint32_t grid = std::min((B + kCosBlocks - 1) / kCosBlocks, kCosGroups);
     {
-        // the cosine kernel, which streams the key sums, also timed alone
+        // the kernel which streams the key sums, also timed alone
         PerfLaunchScope timed(ctx, kPerfMeankCos);
-        ctx_launch(ctx, D == 256 ? meank_cos_kernel<256> : meank_cos_kernel<128>, dim3(grid), dim3(256), 0,
-                   a->k_sum, a->mean_tokens, qv, nq, invq_dev, L, B, cap, a->n_head_kv, layer_cos);
+        const bool q_lds = cos_lds_bytes(L, a->n_head_kv, D, true) <= kCosLds;
+        ctx_launch(ctx, D == 256 ? meank_score_of<256>(a->n_head_kv, q_lds) : meank_score_of<128>(a->n_head_kv, q_lds),
+                   dim3(grid), dim3(kCosWaves * 64u),
+                   static_cast<uint32_t>(cos_lds_bytes(L, a->n_head_kv, D, q_lds)), a->k_sum, a->mean_tokens, qv, nq,
+                   scored, L, B, cap, a->n_head_kv, a->scores);
         if (hip_ok(ctx, hipGetLastError(), "score_meank launch")) {
             timed.ok();
         } else {
@@ -747,9 +811,6 @@ int kvmem_hip_score_meank(kvmem_hip_ctx *ctx, const kvmem_hip_meank_args *a) {
             return KVMEM_HIP_ERR_RUNTIME;
         }
     }
-    constexpr uint32_t kCombineBlocks = 256 / kCombineLayers;
-    meank_combine_kernel<<<(B + kCombineBlocks - 1) / kCombineBlocks, 256, 0, ctx->stream>>>(layer_cos, a->mean_tokens, invq_dev,
-                                                                   L, B, cap, a->n_head_kv, a->scores);
     perf_end(ctx, kPerfScore);
     return hip_ok(ctx, hipGetLastError(), "score_meank launch") ? KVMEM_HIP_OK : KVMEM_HIP_ERR_RUNTIME;
 }

@@ -426,3 +426,46 @@ def test_meank_add_run_edges(ctx, dtype, n, heads, Dh):
     got = acc.cpu().numpy()
     assert np.array_equal(got[:ne].view(np.uint32), ordered_sum(np.concatenate([rows, rows])).view(np.uint32))
     assert np.isnan(got[ne:]).all() and cnt.tolist() == [2 * n, 7]
+
+
+@pytest.mark.parametrize("L_,nb,Hkv,Dh,g", [
+    (1, 1, 1, 128, 1),       # one block of one layer
+    (16, 2051, 2, 128, 4),   # more block groups than workgroups, the last group short
+    (9, 6, 3, 128, 2),       # heads that do not fill a step of four
+    (17, 7, 5, 256, 1),      # steps of two heads, the last half empty
+    (40, 9, 4, 256, 6),      # query vectors past what LDS holds
+    (256, 5, 1, 256, 9),     # the most layers; nine heads to a group
+])
+def test_meank_scores_step_edges(ctx, L_, nb, Hkv, Dh, g):
+    """Mean-K scores against 64 bits.  A cosine's three sums add Dh/16 products
+    in a lane and 16 lanes in a tree; each is within (Dh/16 + 5) * 2^-24 of its
+    terms' sizes, and the query's group sum adds g terms.  Every third layer has
+    no query rows; blocks without keys in some layers hold NaN there."""
+    announce(f"mean-K scores: {L_} layers x {nb} blocks, {Hkv} KV heads x {Dh}, groups of {g}")
+    gen = torch.Generator(device="cuda").manual_seed(L_ + nb)
+    cap = nb + 2
+    ks = torch.randn((L_, cap, Hkv * Dh), generator=gen, device="cuda") * 40
+    mt = torch.randint(1, 129, (L_, cap), generator=gen, device="cuda", dtype=torch.int32)
+    q_sum = torch.randn((L_, Hkv * g * Dh), generator=gen, device="cuda") * 8
+    q_count = [0 if l % 3 == 1 else 1 + l % 7 for l in range(L_)]
+    for l in range(L_):
+        mt[l, (5 * l) % nb] = 0
+        ks[l, (5 * l) % nb] = float("nan")
+    if nb > 2:
+        mt[:, 2] = 0
+        ks[:, 2] = float("nan")
+    scores = torch.full((nb + 1,), -9.0, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    ctx.score_meank(q_sum.data_ptr(), q_count, ks.data_ptr(), mt.data_ptr(), L_, nb, Hkv * g, Hkv, Dh,
+                    scores.data_ptr(), cap)
+    ctx.sync()
+    qc = torch.tensor([float(c) for c in q_count], dtype=torch.float64, device="cuda")
+    qv = q_sum.double().view(L_, Hkv, g, Dh).sum(2) / (qc.clamp(min=1) * g).view(-1, 1, 1)
+    k64 = ks[:, :nb].double().view(L_, nb, Hkv, Dh) / mt[:, :nb].double().clamp(min=1).view(L_, nb, 1, 1)
+    k64 = torch.where((mt[:, :nb] == 0).view(L_, nb, 1, 1), torch.zeros_like(k64), k64)
+    cos = (k64 * qv[:, None]).sum(-1) / (qv.norm(dim=-1)[:, None] * k64.norm(dim=-1) + 1e-6)
+    want = cos.mean(-1)[qc > 0].sum(0) / max(1, int((qc > 0).sum()))
+    want[(mt[:, :nb] == 0).all(0)] = 0.0
+    err = float((scores[:nb].double() - want).abs().max())
+    assert err <= 3 * (Dh / 16 + 5 + g) * 2.0 ** -24, err
+    assert float(scores[nb]) == -9.0
