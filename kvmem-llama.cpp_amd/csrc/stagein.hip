@@ -159,6 +159,7 @@ struct BlockSource {
     uint32_t hadamard;                // Hadamard width (0 = none)
     float hscale;                     // 1 / sqrtf(hadamard)
     uint32_t layer_group;             // layers per workgroup chunk index (RoPE'd K: 4; else 1)
+    uint32_t lw_bits;                 // 64-per-lane kernels: log2 of a workgroup's layer waves
     __device__ void bind(const ArgTables &t) {
         const uint8_t *b = table_base(tables, t);
         layer_dst = reinterpret_cast<const uint8_t *const *>(b + layer_off);
@@ -959,8 +960,9 @@ __global__ __launch_bounds__(256) void quant_scatter_kv_kernel(BlockSource ak, B
 // costs an exchange, a sign and an add per element.  This path gives each
 // lane 64 consecutive elements of a row (two quantization groups) and a
 // wave a unit of 4096 consecutive elements of an operation; a workgroup
-// takes one unit of one block for every layer, wave w the layers w, w + 4,
-// ... (four workgroups per CU hide each other's load latency).  Loads
+// takes one unit of one block for every layer (or some of them, see
+// launch_block_job), wave w the layers w, w + 4, ... (four workgroups per CU
+// hide each other's load latency).  Loads
 // stay coalesced (16 bytes per lane, 1 KiB per wave-wide load) and are
 // redistributed through the wave's LDS with a lane stride of 136 bytes
 // (8-byte halves of consecutive lanes fall on distinct banks on both sides,
@@ -984,7 +986,10 @@ __global__ __launch_bounds__(256) void quant_scatter_kv_kernel(BlockSource ak, B
 //    quantizer scales amax (exactly) and multiplies id by the scale
 //    (exactly) instead.  1/sqrtf(128) and 1/sqrtf(512) are inexact and
 //    scale the elements first, as the reference does.
-//  - RoPE (n_rot 128 and 256): a rotary pair lies in lanes l and
+//  - RoPE, n_rot 64: a rotary pair lies in one lane (x64_rope_f16_lane; 77
+//    blocks x 16 layers of 1024 elements, attn_rot, q8_0: 197 us, 258 with
+//    the 8-elements-per-lane path above that took this shape before).
+//  - RoPE, n_rot 128 and 256: a rotary pair lies in lanes l and
 //    l ^ n_rot/128, and an element becomes fma(partner * sin, t, own * cos),
 //    t = -1 in the first half: the two rounded products and the one rounded
 //    sum of x0*c - x1*s and x0*s + x1*c.  Partners (here and for the
@@ -993,6 +998,7 @@ __global__ __launch_bounds__(256) void quant_scatter_kv_kernel(BlockSource ak, B
 //    all the layers.
 constexpr uint32_t kX64Lane = 136;              // LDS bytes per lane: 128 + 8
 constexpr uint32_t kX64Wave = 64u * kX64Lane;   // LDS bytes of one wave
+constexpr uint32_t kX64FullGrid = 1024;  // workgroups: four per CU
 constexpr uint32_t kX64Groups = 128; // groups of 32 elements in a unit
 
 // cos/sin table of rotary pairs (n_rot = 2 * half, half 64 or 128) in
@@ -1083,6 +1089,21 @@ __device__ inline void x64_rope_f16(float x[64], const uint32_t w[32], const flo
         const float a1 = mix_mul<1>(w[u], cs.z, nz);
         x[2 * u] = __builtin_fmaf(p0, tr, a0);
         x[2 * u + 1] = __builtin_fmaf(p1, tr, a1);
+    }
+}
+
+// RoPE of 64 rotary dims: the head's first 64 elements are one lane's, so the
+// pair of element i is element i + 32 of the same lane.  The same rounded
+// products and sums, without an exchange.
+__device__ inline void x64_rope_f16_lane(float x[64], const uint32_t w[32], const float4 *t) {
+    const float nz = -0.0f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const float4 cs = t[u];  // pairs 2u (x: cos, y: sin) and 2u + 1 (z, w)
+        x[2 * u] = mix_mul<0>(w[u], cs.x, nz) - mix_mul<0>(w[u + 16], cs.y, nz);
+        x[2 * u + 1] = mix_mul<1>(w[u], cs.z, nz) - mix_mul<1>(w[u + 16], cs.w, nz);
+        x[2 * u + 32] = mix_mul<0>(w[u], cs.y, nz) + mix_mul<0>(w[u + 16], cs.x, nz);
+        x[2 * u + 33] = mix_mul<1>(w[u], cs.w, nz) + mix_mul<1>(w[u + 16], cs.z, nz);
     }
 }
 
@@ -1218,15 +1239,27 @@ __device__ inline void x64_quant_lane(const float x[64], float f, float sf, uint
     }
 }
 
-// Workgroup `c` of a block source on this path: unit `sub` (groups g0 ..
-// g0+ng, ng <= 128) of one block, wave w taking layers w, w + 4, ...
-template <int TYPE>
+// Workgroup `c` of a block source on this path: chunk `sub` of one block for
+// layer_group consecutive layers.  LW = 2^lw_bits waves take layers side by
+// side, the w-th the w-th, (w + LW)-th, ...: four, or 2 or 1 where the job has
+// fewer layers; then the chunk has 2 or 4 units, for the other waves (50 blocks
+// of one layer: 17.3 us, 29.1 with three waves idle).
+template <int TYPE, bool ROPE64>
 __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t *lds, uint8_t *tab) {
     constexpr int GB = Fmt<TYPE>::GB;
-    const uint32_t item = c / s.chunks_per_op;
-    const uint32_t sub = c - item * s.chunks_per_op;
+    const uint32_t og = c / s.chunks_per_op;
+    const uint32_t sub = c - og * s.chunks_per_op;
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform per wave
+    const uint32_t lw = 1u << s.lw_bits;
+    uint32_t item = og, lg0 = 0u;  // the block, and the first layer of the workgroup
+    if (s.layer_group < s.n_layers) {
+        const uint32_t layer_groups = (s.n_layers + s.layer_group - 1u) / s.layer_group;
+        item = og / layer_groups;
+        lg0 = (og - item * layer_groups) * s.layer_group;
+    }
+    const uint32_t l0 = lg0 + (wave & (lw - 1u));
+    const uint32_t l1 = min(s.n_layers, lg0 + s.layer_group);
     const uint32_t lane = tid & 63u;
     // the item's fields, read once (uniform): block, slot, tokens, position
     const uint32_t block = s.items[4 * item + 0];
@@ -1235,12 +1268,14 @@ __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t
     ch.pos0 = static_cast<int32_t>(s.items[4 * item + 3]);
     ch.gpr = s.gpr;
     ch.src_stride = s.gpr * 64u;
-    ch.g0 = sub * kX64Groups;
+    const uint32_t cg0 = sub * s.chunk_groups;
     const uint32_t total = s.items[4 * item + 2] * s.gpr;
-    if (ch.g0 >= total) {
-        return;  // uniform: no rows in this unit
+    if (cg0 >= total) {
+        return;  // uniform: no rows in this chunk
     }
-    ch.ng = min(kX64Groups, total - ch.g0);
+    const uint32_t cng = min(s.chunk_groups, total - cg0);
+    ch.g0 = cg0 + (wave >> s.lw_bits) * kX64Groups;
+    ch.ng = ch.g0 < total ? min(kX64Groups, total - ch.g0) : 0u;  // 0: no rows for this wave
     const uint8_t *src0 = s.base + block * s.block_stride;
     const uint64_t dst_off = static_cast<uint64_t>(slot) * s.block_tokens * s.row_bytes;
     const uint32_t nvl = min(64u, ch.ng / 2u);  // lanes with elements (ng is even)
@@ -1251,11 +1286,11 @@ __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t
     const uint32_t e = (ch.g0 + 2u * lane) * 32u;
     const uint32_t row = e / E;
     const uint32_t d0 = (e - row * E) & (s.head_dim - 1u);
-    const uint32_t row0 = ch.g0 / ch.gpr;
+    const uint32_t row0 = cg0 / ch.gpr;  // the table holds the rows of the whole chunk
     const uint32_t half = s.n_rot / 2u;
     const X64Tab tg = x64_tab_geom(half);
     if (half != 0u) {
-        const uint32_t rows = (ch.g0 + ch.ng - 1u) / ch.gpr - row0 + 1u;
+        const uint32_t rows = (cg0 + cng - 1u) / ch.gpr - row0 + 1u;
         for (uint32_t i = tid; i < rows * half; i += blockDim.x) {
             const uint32_t r = i / half;
             const uint32_t j = i - r * half;
@@ -1292,7 +1327,10 @@ __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t
     uint8_t *wr = wl + (lane >> 3) * kX64Lane + (lane & 7u) * 16u;
     const uint8_t *rd = wl + lane * kX64Lane;
 
-    for (uint32_t l = wave; l < s.n_layers; l += 4u) {
+    if (ch.ng == 0u) {
+        return;
+    }
+    for (uint32_t l = l0; l < l1; l += lw) {
         ch.src = src0 + l * s.layer_stride;  // the same rows of layer l
         ch.dst = const_cast<uint8_t *>(s.layer_dst[l]) + dst_off;
         uint4 v[8];
@@ -1317,7 +1355,11 @@ __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t
         // the first operation on each element widens it
         float x[64];
         if (half != 0u && rot) {
-            x64_rope_f16(x, w, trow, tr, rope_src);
+            if constexpr (ROPE64) {
+                x64_rope_f16_lane(x, w, trow);
+            } else {
+                x64_rope_f16(x, w, trow, tr, rope_src);
+            }
         } else if (first_sum) {  // Hadamard span 1 with the scale carried to the quantizer
 #pragma unroll
             for (int m = 0; m < 32; ++m) {
@@ -1400,16 +1442,16 @@ __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t
     }
 }
 
-template <int TYPE>
+template <int TYPE, bool ROPE64>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void x64_kernel(BlockSource a,
                                                                                             ArgTables t) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kX64Wave];
     BlockSource s = a;
     s.bind(t);
-    x64_unit_layers<TYPE>(s, xcd_chunk(blockIdx.x, gridDim.x), lds, reinterpret_cast<uint8_t *>(rope_tab4));
+    x64_unit_layers<TYPE, ROPE64>(s, xcd_chunk(blockIdx.x, gridDim.x), lds, reinterpret_cast<uint8_t *>(rope_tab4));
 }
 
-template <int TK, int TV>
+template <int TK, int TV, bool ROPE64>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void x64_kv_kernel(BlockSource ak, BlockSource av, uint32_t n_k, ArgTables t) {
     BlockSource sk = ak, sv = av;
     sk.bind(t);
@@ -1418,9 +1460,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void x
     const uint32_t c = xcd_chunk(blockIdx.x, gridDim.x);
     uint8_t *tab = reinterpret_cast<uint8_t *>(rope_tab4);
     if (c < n_k) {
-        x64_unit_layers<TK>(sk, c, lds, tab);
+        x64_unit_layers<TK, ROPE64>(sk, c, lds, tab);
     } else {
-        x64_unit_layers<TV>(sv, c - n_k, lds, tab);
+        x64_unit_layers<TV, false>(sv, c - n_k, lds, tab);
     }
 }
 
@@ -1611,12 +1653,12 @@ static int resolve_xf(kvmem_hip_ctx *ctx, const kvmem_hip_pool *pool, uint32_t e
     // the reference's scale, 1.0f / sqrtf((float) nrot) (stagein.cu:557)
     out.hscale_k = out.had_k ? 1.0f / sqrtf(static_cast<float>(out.had_k)) : 1.0f;
     out.hscale_v = out.had_v ? 1.0f / sqrtf(static_cast<float>(out.had_v)) : 1.0f;
-    // The 64-elements-per-lane kernels hold a rotary pair in lanes l and
-    // l ^ n_rot/128 (n_rot 128, 256), and F16 rows only without cross-lane
+    // The 64-elements-per-lane kernels hold a rotary pair in one lane (n_rot
+    // 64) or in lanes l and l ^ n_rot/128 (n_rot 128, 256), and F16 rows only without cross-lane
     // butterflies (width 64); other shapes take the 8-elements-per-lane
     // kernels.
     const uint32_t half = out.n_rot / 2;
-    out.lane64 = (half == 0 || half == 64 || half == 128) &&
+    out.lane64 = (half == 0 || half == 32 || half == 64 || half == 128) &&
                  ek % 64 == 0 && (!want_v || ev % 64 == 0) &&
                  (pool->type_k != KVMEM_TYPE_F16 || out.had_k <= 64) &&
                  (!want_v || pool->type_v != KVMEM_TYPE_F16 || out.had_v <= 64);
@@ -1687,9 +1729,10 @@ static BlockSource make_block_source(int type, const uint8_t *base, uint64_t blo
     s.n_rot = is_k ? xp.n_rot : 0u;
     s.hadamard = is_k ? xp.had_k : xp.had_v;
     s.hscale = is_k ? xp.hscale_k : xp.hscale_v;
-    if (xp.lane64) {  // one workgroup per unit of 128 groups, every layer
-        s.chunk_groups = kX64Groups;
-        s.chunks_per_op = (block_tokens * s.gpr + kX64Groups - 1) / kX64Groups;
+    if (xp.lane64) {  // units of 128 groups, every layer (launch_block_job may split them)
+        s.lw_bits = n_layers >= 4u ? 2u : n_layers >= 2u ? 1u : 0u;
+        s.chunk_groups = kX64Groups << (2u - s.lw_bits);
+        s.chunks_per_op = (block_tokens * s.gpr + s.chunk_groups - 1) / s.chunk_groups;
         s.layer_group = n_layers;
     } else {
         s.layer_group = (xp.on && s.n_rot) ? kRopeLayerGroup : 1u;
@@ -1711,17 +1754,30 @@ static size_t x64_tab_bytes(const BlockSource &s) {
     return static_cast<size_t>(chunk_rows_of(s.gpr, s.chunk_groups)) * x64_tab_geom(s.n_rot / 2).RS * 16u;
 }
 
-template <int TK>
+template <int TK, bool ROPE64>
 static bool launch_x64_v(kvmem_hip_ctx *ctx, int tv, uint32_t grid, size_t tb, const BlockSource &sk,
-                         const BlockSource &sv, uint32_t n_k, const ArgTables &args) {
+                         const BlockSource *sv, uint32_t n_k, const ArgTables &args) {
+    const dim3 g(grid), b(256);
+    const uint32_t lds = static_cast<uint32_t>(tb);
+    if (!sv) {
+        ctx_launch(ctx, x64_kernel<TK, ROPE64>, g, b, lds, sk, args);
+        return true;
+    }
     switch (tv) {
-        case KVMEM_TYPE_Q8_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q8_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, sv, n_k, args); break;
-        case KVMEM_TYPE_Q4_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q4_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, sv, n_k, args); break;
-        case KVMEM_TYPE_Q5_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q5_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, sv, n_k, args); break;
-        case KVMEM_TYPE_F16: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_F16>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, sv, n_k, args); break;
+        case KVMEM_TYPE_Q8_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q8_0, ROPE64>, g, b, lds, sk, *sv, n_k, args); break;
+        case KVMEM_TYPE_Q4_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q4_0, ROPE64>, g, b, lds, sk, *sv, n_k, args); break;
+        case KVMEM_TYPE_Q5_0: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_Q5_0, ROPE64>, g, b, lds, sk, *sv, n_k, args); break;
+        case KVMEM_TYPE_F16: ctx_launch(ctx, x64_kv_kernel<TK, KVMEM_TYPE_F16, ROPE64>, g, b, lds, sk, *sv, n_k, args); break;
         default: fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED, "stage-in: unsupported V type"); return false;
     }
     return true;
+}
+
+template <int TK>
+static bool launch_x64_k(kvmem_hip_ctx *ctx, int tv, uint32_t grid, size_t tb, const BlockSource &sk,
+                         const BlockSource *sv, uint32_t n_k, const ArgTables &args) {
+    return sk.n_rot == 64u ? launch_x64_v<TK, true>(ctx, tv, grid, tb, sk, sv, n_k, args)
+                           : launch_x64_v<TK, false>(ctx, tv, grid, tb, sk, sv, n_k, args);
 }
 
 // The job on the 64-elements-per-lane kernels (K chunks first, then V).
@@ -1735,30 +1791,36 @@ static bool launch_x64(kvmem_hip_ctx *ctx, int tk, int tv, uint32_t n_k, uint32_
     }
     const size_t tb = x64_tab_bytes(sk);  // only K is RoPE'd
     const uint32_t grid = n_k + n_v;
-    bool ok = true;
-    if (sv) {
-        switch (tk) {
-            case KVMEM_TYPE_Q8_0: ok = launch_x64_v<KVMEM_TYPE_Q8_0>(ctx, tv, grid, tb, sk, *sv, n_k, args); break;
-            case KVMEM_TYPE_Q4_0: ok = launch_x64_v<KVMEM_TYPE_Q4_0>(ctx, tv, grid, tb, sk, *sv, n_k, args); break;
-            case KVMEM_TYPE_Q5_0: ok = launch_x64_v<KVMEM_TYPE_Q5_0>(ctx, tv, grid, tb, sk, *sv, n_k, args); break;
-            case KVMEM_TYPE_F16: ok = launch_x64_v<KVMEM_TYPE_F16>(ctx, tv, grid, tb, sk, *sv, n_k, args); break;
-            default: fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED, "stage-in: unsupported K type"); return false;
-        }
-    } else {
-        switch (tk) {
-            case KVMEM_TYPE_Q8_0: ctx_launch(ctx, x64_kernel<KVMEM_TYPE_Q8_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, args); break;
-            case KVMEM_TYPE_Q4_0: ctx_launch(ctx, x64_kernel<KVMEM_TYPE_Q4_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, args); break;
-            case KVMEM_TYPE_Q5_0: ctx_launch(ctx, x64_kernel<KVMEM_TYPE_Q5_0>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, args); break;
-            case KVMEM_TYPE_F16: ctx_launch(ctx, x64_kernel<KVMEM_TYPE_F16>, dim3(grid), dim3(256), static_cast<uint32_t>(tb), sk, args); break;
-            default: fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED, "stage-in: unsupported K type"); return false;
-        }
+    bool ok = false;
+    switch (tk) {
+        case KVMEM_TYPE_Q8_0: ok = launch_x64_k<KVMEM_TYPE_Q8_0>(ctx, tv, grid, tb, sk, sv, n_k, args); break;
+        case KVMEM_TYPE_Q4_0: ok = launch_x64_k<KVMEM_TYPE_Q4_0>(ctx, tv, grid, tb, sk, sv, n_k, args); break;
+        case KVMEM_TYPE_Q5_0: ok = launch_x64_k<KVMEM_TYPE_Q5_0>(ctx, tv, grid, tb, sk, sv, n_k, args); break;
+        case KVMEM_TYPE_F16: ok = launch_x64_k<KVMEM_TYPE_F16>(ctx, tv, grid, tb, sk, sv, n_k, args); break;
+        default: fail(ctx, KVMEM_HIP_ERR_UNSUPPORTED, "stage-in: unsupported K type"); return false;
     }
     return ok && hip_ok(ctx, hipGetLastError(), "stage-in transform kernel launch");
 }
 
-static int launch_block_job(kvmem_hip_ctx *ctx, int type_k, const BlockSource &sk, int type_v,
-                            const BlockSource *sv, uint32_t n_items, const XfParams &xp,
+static int launch_block_job(kvmem_hip_ctx *ctx, int type_k, const BlockSource &k, int type_v,
+                            const BlockSource *v, uint32_t n_items, const XfParams &xp,
                             const ArgTables &args) {
+    BlockSource sk = k, sv_copy = v ? *v : BlockSource{};
+    const BlockSource *sv = v ? &sv_copy : nullptr;
+    if (xp.lane64) {
+        // A workgroup takes every layer of a unit (one cos/sin table), a wave
+        // one after the other.  Below four workgroups per CU that leaves the
+        // chip empty, and the layers are split over more workgroups (16
+        // layers, RoPE 256 and attn_rot: one block 12.3 us, 35.7 unsplit; four
+        // 16.0 and 37.3).  Splitting also where 1536 workgroups fill the
+        // chip, for an even end, costs more tables than it gains (24 blocks:
+        // 63.9 us, 67.3 split).
+        while (sk.layer_group > 4u &&
+               block_job_chunks(sk, n_items) + (sv ? block_job_chunks(*sv, n_items) : 0) < kX64FullGrid) {
+            sk.layer_group = ((sk.layer_group + 1u) / 2u + 3u) / 4u * 4u;
+            sv_copy.layer_group = sk.layer_group;
+        }
+    }
     const uint64_t nk = block_job_chunks(sk, n_items);
     const uint64_t nv = sv ? block_job_chunks(*sv, n_items) : 0;
     if (nk + nv > 0x7fffffffu) {

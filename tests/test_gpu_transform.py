@@ -222,3 +222,21 @@ def test_engine_rope_attn_rot(oracle):
                     got = pool[s * T:(s + 1) * T]
                     assert np.array_equal(got, want), f"layer {layer} {'KV'[which]} block {b}: {first_diff(got, want)}"
         c.close()
+
+
+@pytest.mark.parametrize("L,D,hkv,n_rot,hk,tk,tv,last", [
+    (1, 128, 1, 64, 128, kv.TYPE_Q8_0, kv.TYPE_Q8_0, 3),     # four units per chunk of 128 rows: the largest table
+    (1, 256, 4, 256, 256, kv.TYPE_Q4_0, kv.TYPE_Q8_0, 9),    # one layer: four units side by side, some without rows
+    (2, 256, 4, 64, 256, kv.TYPE_Q5_0, kv.TYPE_Q5_0, 101),   # two layers beside two units
+    (3, 128, 8, 64, 64, kv.TYPE_F16, kv.TYPE_Q4_0, 4),
+    (5, 128, 4, 64, 128, kv.TYPE_Q8_0, kv.TYPE_Q4_0, 0),     # layers split 4 + 1
+    (9, 256, 2, 256, 256, kv.TYPE_Q8_0, kv.TYPE_Q8_0, 33),   # 4 + 4 + 1
+    (16, 64, 2, 64, 64, kv.TYPE_Q8_0, kv.TYPE_Q8_0, 65),     # a head within one lane
+])
+def test_transform_layer_splits(ctx, oracle, L, D, hkv, n_rot, hk, tk, tv, last):
+    """The 64-elements-per-lane kernel over layer counts that leave waves to
+    further units and jobs small enough to split the layers, rotary pairs
+    within a lane included."""
+    announce(f"{L} layers, head_dim {D} x {hkv}, n_rot {n_rot}, Hadamard {hk}, K={tk} V={tv}, last {last}")
+    run_case(ctx, oracle, L=L, B=3, Hkv=hkv, D=D, type_k=tk, type_v=tv, n_rot=n_rot, had_k=hk, had_v=64,
+             ids=[2, 0], slots=[3, 1], n_slots=4, last=last, pos0=[1 << 18, 77], seed=L + D + last)
