@@ -9,13 +9,17 @@
 // therefore distinct, and the selection is "the `need` largest keys".
 // Forced ids get key 0, below every finite score, and a bit in a mask.
 //
-// The need-th largest key is found by radix select, eight passes of 8 bits
-// from the top: each pass histograms the digit of the keys that match the
-// digits fixed so far, and one wave picks the digit where the running count
-// from the top reaches the remaining rank.  Winners are the keys at or above
-// that threshold; they and the forced ids are compacted in ascending id
-// order with a workgroup prefix sum, which is the window order of
-// KvMemStore::pick_topk_ungrouped (kvmem_store.cpp:618-622).
+// The need-th largest key is found by radix select, in passes of 8 bits from
+// the highest bit in which any two scores differ: each pass histograms the
+// digit of the keys that match the digits fixed so far, and one wave picks the
+// digit where the running count from the top reaches the remaining rank.
+// (Scores of one call share their sign and most of their exponent.  A pass
+// over those bits puts nearly every key into one histogram word, where the
+// LDS atomics of a wave queue up.  2048 scores: 8.3 us, 10.0 with passes from
+// the top bit and four barriers each; 8192 scores: 12.7 and 21.0.)
+// Winners are the keys at or above that threshold; they and the forced ids are
+// compacted in ascending id order with a workgroup prefix sum, which is the
+// window order of KvMemStore::pick_topk_ungrouped (kvmem_store.cpp:618-622).
 //
 // The selection goes straight to coherent pinned host memory: the ids are
 // compacted in LDS, one wave writes them out with coalesced stores, and a
@@ -85,6 +89,130 @@ __device__ inline uint32_t block_inclusive_scan(uint32_t v, uint32_t *wave_tot) 
     return v + (wave > 0 ? wave_tot[wave - 1] : 0u);
 }
 
+// OR over the 64 lanes of a wave (DPP within a 16-lane row, then the row
+// swaps); every lane must be active.
+__device__ inline uint32_t wave_or(uint32_t x) {
+    x |= __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false);
+    x |= __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false);
+    x |= __builtin_amdgcn_update_dpp(x, x, 0x124, 0xF, 0xF, false);
+    x |= __builtin_amdgcn_update_dpp(x, x, 0x128, 0xF, 0xF, false);
+    const auto s16 = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = s16[0] | s16[1];
+    const auto s32 = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return s32[0] | s32[1];
+}
+
+struct RadixShared {
+    uint32_t hist[256];
+    uint32_t ones[kTopkWaves], zeros[kTopkWaves];  // per wave: OR of the score words, and of their complements
+    uint64_t prefix;
+    uint32_t rank;
+    uint32_t alone;
+};
+
+// The key of rank `need` (from the largest; need > 0, at most the number of
+// candidates) among key_of(0 .. n), 0 = no candidate, on the bits of `mask`: a
+// candidate is of that rank or better when its key on those bits is >= the
+// value returned.  Keys are unique, so once the digit holding the rank has a
+// single key the digits decided so far order every other key against it, and
+// the later passes are skipped.  Called by the whole workgroup.
+template <class KeyOf>
+__device__ inline uint64_t radix_threshold(uint32_t n, uint32_t need, bool tie_lower, const KeyOf &key_of,
+                                           RadixShared &sh, uint64_t &mask) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u;
+    uint32_t ones = 0u, zeros = 0u;
+    for (uint32_t i = tid; i < n; i += kTopkThreads) {
+        const uint64_t k = key_of(i);
+        if (k != 0ull) {
+            ones |= static_cast<uint32_t>(k >> 32);
+            zeros |= ~static_cast<uint32_t>(k >> 32);
+        }
+    }
+    ones = wave_or(ones);
+    zeros = wave_or(zeros);
+    if (lane == 0u) {
+        sh.ones[tid >> 6] = ones;
+        sh.zeros[tid >> 6] = zeros;
+    }
+    if (tid < 256u) {
+        sh.hist[tid] = 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kTopkWaves; ++w) {
+        ones |= sh.ones[w];
+        zeros |= sh.zeros[w];
+    }
+    // key bits still open: from the scores' highest differing bit down
+    const uint32_t differ = ones & zeros;
+    const uint32_t id_bits = n > 1u ? 32u - static_cast<uint32_t>(__clz(static_cast<int>(n - 1u))) : 0u;
+    uint32_t open = 32u + (differ ? 32u - static_cast<uint32_t>(__clz(static_cast<int>(differ))) : 0u);
+    mask = open == 64u ? 0ull : ~0ull << open;
+    uint64_t prefix = (static_cast<uint64_t>(ones) << 32) & mask;
+    uint32_t rank = need;  // still to find among keys matching `prefix`
+    while (true) {
+        if (open == 32u) {  // equal scores: the id word, of which only id_bits differ
+            const uint64_t same = 0xffffffffull & (~0ull << id_bits);
+            mask |= same;
+            prefix |= tie_lower ? same : 0ull;
+            open = id_bits;
+        }
+        if (open == 0u) {
+            break;
+        }
+        const uint32_t width = min(8u, open > 32u ? open - 32u : open);
+        const uint32_t shift = open - width;
+        const uint32_t digits = (1u << width) - 1u;
+        for (uint32_t i = tid; i < n; i += kTopkThreads) {
+            const uint64_t k = key_of(i);
+            if (k != 0ull && (k & mask) == prefix) {
+                atomicAdd(&sh.hist[static_cast<uint32_t>(k >> shift) & digits], 1u);
+            }
+        }
+        __syncthreads();
+        if (tid < 64u) {
+            // lane owns digits 4*lane .. 4*lane+3; above(d) = count of
+            // matching keys whose digit exceeds d
+            uint32_t c[4];
+            uint32_t own = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                c[j] = sh.hist[4u * lane + j];
+                sh.hist[4u * lane + j] = 0u;  // for the next pass
+                own += c[j];
+            }
+            uint32_t suffix = own;  // sum over lanes >= this one
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t t = __shfl_down(suffix, off, 64);
+                if (lane + off < 64u) {
+                    suffix += t;
+                }
+            }
+            uint32_t above = suffix - own;  // digits of higher lanes
+#pragma unroll
+            for (int j = 3; j >= 0; --j) {
+                if (above < rank && rank <= above + c[j]) {
+                    sh.prefix = prefix | (static_cast<uint64_t>(4u * lane + j) << shift);
+                    sh.rank = rank - above;
+                    sh.alone = c[j] == 1u ? 1u : 0u;
+                }
+                above += c[j];
+            }
+        }
+        __syncthreads();  // (the next pass writes these only after its own first barrier)
+        prefix = sh.prefix;
+        rank = sh.rank;
+        mask |= static_cast<uint64_t>(digits) << shift;
+        open = shift;
+        if (sh.alone != 0u) {
+            break;
+        }
+    }
+    return prefix;
+}
+
 // `forced` is a device list, or null with the ids in `forced_inline`.
 // `out` (host-mapped) receives the ids at [0, count) and the count at [n];
 // `done` is set to `epoch` once both are visible to the host.  `dev_out`,
@@ -99,13 +227,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_kernel(const float *scores,
                                                             uint32_t *dev_out) {
     __shared__ uint64_t keys[kTopkMaxN];
     __shared__ uint32_t forced_bits[kTopkMaxN / 32];
-    __shared__ uint32_t hist[256];
     __shared__ uint32_t wave_tot[kTopkWaves];
-    __shared__ uint64_t s_prefix;
-    __shared__ uint32_t s_rank;
-    __shared__ uint32_t s_alone;
+    __shared__ RadixShared radix;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
     const bool tl = tie_lower != 0;
 
     for (uint32_t i = tid; i < n; i += kTopkThreads) {
@@ -122,72 +246,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_kernel(const float *scores,
     }
     __syncthreads();
 
-    // ---- radix select: threshold = the need-th largest candidate key.
-    // Keys are unique, so once the digit holding that rank has a single key
-    // it is the threshold, and the digits decided so far (`mask`) order
-    // every other key against it: the later passes are skipped.
-    uint64_t prefix = 0ull;
     uint64_t mask = 0ull;
-    uint32_t rank = need;  // rank still to find among keys matching `prefix`
-    if (need > 0u) {
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            if (tid < 256u) {
-                hist[tid] = 0u;
-            }
-            if (tid == 0u) {
-                s_alone = 0u;
-            }
-            __syncthreads();
-            for (uint32_t i = tid; i < n; i += kTopkThreads) {
-                const uint64_t k = keys[i];
-                if (k != 0ull && (k & mask) == prefix) {
-                    atomicAdd(&hist[static_cast<uint32_t>(k >> shift) & 255u], 1u);
-                }
-            }
-            __syncthreads();
-            if (tid < 64u) {
-                // lane owns digits 4*lane .. 4*lane+3; above(d) = count of
-                // matching keys whose digit exceeds d
-                uint32_t c[4];
-                uint32_t own = 0u;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    c[j] = hist[4u * lane + j];
-                    own += c[j];
-                }
-                uint32_t suffix = own;  // sum over lanes >= this one
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t t = __shfl_down(suffix, off, 64);
-                    if (lane + off < 64u) {
-                        suffix += t;
-                    }
-                }
-                uint32_t above = suffix - own;  // digits of higher lanes
-#pragma unroll
-                for (int j = 3; j >= 0; --j) {
-                    if (above < rank && rank <= above + c[j]) {
-                        s_prefix = prefix | (static_cast<uint64_t>(4u * lane + j) << shift);
-                        s_rank = rank - above;
-                        s_alone = c[j] == 1u ? 1u : 0u;
-                    }
-                    above += c[j];
-                }
-            }
-            __syncthreads();
-            prefix = s_prefix;
-            rank = s_rank;
-            mask |= 0xffull << shift;
-            const bool alone = s_alone != 0u;
-            __syncthreads();  // s_prefix / s_alone / hist are rewritten by the next pass
-            if (alone) {
-                break;
-            }
-        }
-    }
-    // the key of rank `need`, on the bits decided (all 64 unless it stood
-    // alone earlier): a candidate wins when its key on those bits is >= it
-    const uint64_t threshold = prefix;
+    const uint64_t threshold =
+        need > 0u ? radix_threshold(n, need, tl, [&](uint32_t i) { return keys[i]; }, radix, mask) : 0ull;
 
     // ---- ordered compaction: thread t owns ids [t*seg, (t+1)*seg)
     const uint32_t seg = (n + kTopkThreads - 1) / kTopkThreads;
@@ -253,13 +314,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_stream_kernel(
     uint32_t n_forced, uint32_t need, int tie_lower, uint32_t *out, uint32_t *done, uint32_t epoch,
     uint32_t *dev_out) {
     __shared__ uint32_t forced_bits[kTopkStreamMaxN / 32];
-    __shared__ uint32_t hist[256];
     __shared__ uint32_t wave_tot[kTopkWaves];
-    __shared__ uint64_t s_prefix;
-    __shared__ uint32_t s_rank;
-    __shared__ uint32_t s_alone;
+    __shared__ RadixShared radix;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
     const bool tl = tie_lower != 0;
     for (uint32_t w = tid; w < (n + 31u) / 32u; w += kTopkThreads) {
         forced_bits[w] = 0u;
@@ -273,66 +330,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_stream_kernel(
     auto is_forced = [&](uint32_t i) -> bool { return (forced_bits[i >> 5] >> (i & 31u)) & 1u; };
     auto key_of = [&](uint32_t i) -> uint64_t { return is_forced(i) ? 0ull : rank_key(scores[i], i, tl); };
 
-    // the same radix select as topk_kernel's, its passes skipped once the
-    // threshold key stands alone in its digit
-    uint64_t prefix = 0ull;
     uint64_t mask = 0ull;
-    uint32_t rank = need;
-    if (need > 0u) {
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            if (tid < 256u) {
-                hist[tid] = 0u;
-            }
-            if (tid == 0u) {
-                s_alone = 0u;
-            }
-            __syncthreads();
-            for (uint32_t i = tid; i < n; i += kTopkThreads) {
-                const uint64_t k = key_of(i);
-                if (k != 0ull && (k & mask) == prefix) {
-                    atomicAdd(&hist[static_cast<uint32_t>(k >> shift) & 255u], 1u);
-                }
-            }
-            __syncthreads();
-            if (tid < 64u) {
-                uint32_t c[4];
-                uint32_t own = 0u;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    c[j] = hist[4u * lane + j];
-                    own += c[j];
-                }
-                uint32_t suffix = own;
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t t = __shfl_down(suffix, off, 64);
-                    if (lane + off < 64u) {
-                        suffix += t;
-                    }
-                }
-                uint32_t above = suffix - own;
-#pragma unroll
-                for (int j = 3; j >= 0; --j) {
-                    if (above < rank && rank <= above + c[j]) {
-                        s_prefix = prefix | (static_cast<uint64_t>(4u * lane + j) << shift);
-                        s_rank = rank - above;
-                        s_alone = c[j] == 1u ? 1u : 0u;
-                    }
-                    above += c[j];
-                }
-            }
-            __syncthreads();
-            prefix = s_prefix;
-            rank = s_rank;
-            mask |= 0xffull << shift;
-            const bool alone = s_alone != 0u;
-            __syncthreads();
-            if (alone) {
-                break;
-            }
-        }
-    }
-    const uint64_t threshold = prefix;  // on the bits in `mask`
+    const uint64_t threshold = need > 0u ? radix_threshold(n, need, tl, key_of, radix, mask) : 0ull;
     auto chosen = [&](uint32_t i) -> bool {
         if (is_forced(i)) {
             return true;

@@ -169,3 +169,37 @@ def test_topk_many_forced_ids_uploaded(ctx, oracle, n, tie_lower):
     torch.cuda.synchronize()
     got = ctx.topk(d.data_ptr(), n, need, forced=forced + forced[:20], tie_lower_index=tie_lower)
     assert got == want
+
+
+def radix_scores(kind: str, n: int) -> np.ndarray:
+    rng = np.random.default_rng(n)
+    if kind == "equal":              # no score bit differs: the ids decide
+        return np.full(n, -3.25, np.float32)
+    if kind == "last_bit":           # only the lowest bit does
+        return (np.float32(1.5).view(np.uint32) | rng.integers(0, 2, n, dtype=np.uint32)).view(np.float32)
+    if kind == "signs":              # the highest does
+        return np.where(rng.random(n) < 0.5, -1, 1).astype(np.float32) * rng.random(n).astype(np.float32)
+    if kind == "extremes":
+        s = rng.standard_normal(n).astype(np.float32)
+        s[::3] = np.finfo(np.float32).max
+        s[1::7] = -np.finfo(np.float32).max
+        s[2::5] = -0.0
+        s[3::11] = 1e-42             # subnormal
+        return s
+    return (6.0 + 0.25 * rng.standard_normal(n)).astype(np.float32)  # as block scores are
+
+
+@pytest.mark.parametrize("kind", ["equal", "last_bit", "signs", "extremes", "scores"])
+@pytest.mark.parametrize("n,need", [(2, 1), (2, 0), (64, 63), (257, 1), (1025, 300), (16384, 16383), (16385, 5),
+                                    (20000, 19999)])
+@pytest.mark.parametrize("tie_lower", [True, False])
+def test_topk_radix_windows(ctx, oracle, kind, n, need, tie_lower):
+    """The radix select starts at the highest bit in which two scores differ:
+    scores that differ nowhere, in one end or in the other of their bits, one
+    candidate up to all of them, both kernels."""
+    announce(f"radix: {kind} n={n} need={need} tie_lower={tie_lower}")
+    s = radix_scores(kind, n)
+    d = dev(s)
+    torch.cuda.synchronize()
+    got = ctx.topk(d.data_ptr(), n, need, forced=[0], tie_lower_index=tie_lower)
+    assert got == oracle.pick_topk(s.astype(np.float64), need + 1, sink=1, tie_lower_index=tie_lower)
