@@ -454,34 +454,41 @@ __global__ __launch_bounds__(WR * 64, score_occupancy(D, RT)) void score_kernel(
 // A workgroup takes 16 blocks; 16 threads per block take the layers l,
 // l + 16, ... and issue a layer's partial maxima as one batch of loads.
 // After the barrier one thread per block reduces its layers in layer order,
-// again loading 16 layers per batch.  The arithmetic is the plain loops'
-// (a max chain in (slice, head) order, an ordered float sum), so batching
-// changes no bit.
+// from LDS (up to kFoldLayers layers; from memory beyond).  The arithmetic is
+// the plain loops' (a max chain in (slice, head) order, an ordered float sum),
+// so batching changes no bit.  Latency-bound: 2 x 12 blocks 2.1 us, 3.8 with the
+// layer scores read back from memory and a division per partial (16 x 2048
+// blocks: 5.2 and 6.0).
 constexpr uint32_t kFoldBlocks = 16;
 constexpr uint32_t kFoldLanes = 256 / kFoldBlocks;
 constexpr uint32_t kFoldBatch = 16;
+constexpr uint32_t kFoldLayers = 64;
+static_assert(kFoldLayers % kFoldBatch == 0, "whole batches from LDS");
 
 __global__ __launch_bounds__(256) void score_fold_kernel(const float *partial, uint32_t S,
                                                          uint32_t L, uint32_t Hkv, uint32_t B,
                                                          float *layer_scores, int mode,
                                                          float *scores) {
+    __shared__ float of_layer[kFoldLayers][kFoldBlocks];
     const uint32_t bl = threadIdx.x % kFoldBlocks;
     const uint32_t lane = threadIdx.x / kFoldBlocks;
     const uint32_t b = blockIdx.x * kFoldBlocks + bl;
     const uint32_t per_layer = S * Hkv;
+    const uint64_t slice_step = (static_cast<uint64_t>(L) - 1u) * Hkv * B;  // from a slice's last head to the next's first
     if (b < B) {
         for (uint32_t l = lane; l < L; l += kFoldLanes) {
             float best = -FLT_MAX;
+            uint32_t h = 0;  // head of the next partial (uniform)
+            uint64_t at = static_cast<uint64_t>(l) * Hkv * B + b;
             for (uint32_t i0 = 0; i0 < per_layer; i0 += kFoldBatch) {
                 float v[kFoldBatch];
 #pragma unroll
                 for (uint32_t j = 0; j < kFoldBatch; ++j) {
-                    const uint32_t i = i0 + j;
-                    v[j] = -FLT_MAX;
-                    if (i < per_layer) {
-                        const uint32_t sl = i / Hkv;
-                        const uint32_t h = i - sl * Hkv;
-                        v[j] = partial[((static_cast<uint64_t>(sl) * L + l) * Hkv + h) * B + b];
+                    v[j] = i0 + j < per_layer ? partial[at] : -FLT_MAX;
+                    at += B;
+                    if (++h == Hkv) {
+                        h = 0;
+                        at += slice_step;
                     }
                 }
 #pragma unroll
@@ -490,6 +497,9 @@ __global__ __launch_bounds__(256) void score_fold_kernel(const float *partial, u
                 }
             }
             layer_scores[static_cast<uint64_t>(l) * B + b] = best;
+            if (l < kFoldLayers) {
+                of_layer[l][bl] = best;
+            }
         }
     }
     __syncthreads();
@@ -500,9 +510,16 @@ __global__ __launch_bounds__(256) void score_fold_kernel(const float *partial, u
     float acc = max_mode ? -FLT_MAX : 0.0f;
     for (uint32_t l0 = 0; l0 < L; l0 += kFoldBatch) {
         float v[kFoldBatch];
+        if (l0 < kFoldLayers) {  // (a whole batch; what lies past L is not used)
 #pragma unroll
-        for (uint32_t j = 0; j < kFoldBatch; ++j) {
-            v[j] = l0 + j < L ? layer_scores[static_cast<uint64_t>(l0 + j) * B + b] : 0.0f;
+            for (uint32_t j = 0; j < kFoldBatch; ++j) {
+                v[j] = of_layer[l0 + j][bl];
+            }
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < kFoldBatch; ++j) {
+                v[j] = l0 + j < L ? layer_scores[static_cast<uint64_t>(l0 + j) * B + b] : 0.0f;
+            }
         }
 #pragma unroll
         for (uint32_t j = 0; j < kFoldBatch; ++j) {

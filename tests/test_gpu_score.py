@@ -250,3 +250,20 @@ def test_score_tile_edges(ctx, D, g, Tq, T, B, last_T):
     tol = (D + 4) * 2.0 ** -24
     assert np.all(np.abs(ls - want) <= tol * np.abs(want))
     assert np.all(np.abs(s - want.mean(0)) <= 2 * tol * np.abs(want.mean(0)))
+
+
+@pytest.mark.parametrize("L", [64, 65, 90])
+@pytest.mark.parametrize("mode", [kv.LAYER_MEAN, kv.LAYER_MAX])
+def test_score_fold_past_lds_layers(ctx, L, mode):
+    """Layer counts at and past the 64 the fold keeps in LDS, an odd number of
+    partial maxima: the block score is the f32 reduction, in layer order, of
+    the layer scores the same call returns."""
+    announce(f"fold: {L} layers, mode {mode}")
+    k, _, q = workloads.scoring_tensors(torch, "cuda", L=L, B=17, Tq=3, seed=L, T=16, Hkv=3, Hq=3, D=128)
+    s, ls = run_score(ctx, k, q, kv.TYPE_BF16, 3, 3, 128, reduce=mode)
+    want = np.float32(-np.finfo(np.float32).max if mode == kv.LAYER_MAX else 0) * np.ones(17, np.float32)
+    for row in ls.astype(np.float32):
+        want = np.maximum(want, row) if mode == kv.LAYER_MAX else want + row
+    if mode == kv.LAYER_MEAN:
+        want = want / np.float32(L)
+    assert np.array_equal(s.astype(np.float32).view(np.uint32), want.astype(np.float32).view(np.uint32))
