@@ -2030,7 +2030,16 @@ static void chain_table(const kvmem_hip_pool *pool, bool want_v, const std::vect
 // first is saved to scratch beforehand, as build_chains (move_plan.cpp)
 // does on the host.
 constexpr uint32_t kPlanThreads = 1024;
-constexpr uint32_t kChainRows = 64;  // chain segments the device plan's walk runs side by side
+// Grid rows of the device plan's walk, which is launched before the number of
+// segments is known: a quarter of the largest selection, at most 64.  Turns
+// of neighbouring selections make about that many chains (60 segments of 256
+// selected blocks with 30 % new, 13 of 64); further segments take turns.  An
+// empty row costs the dispatch of its workgroups, a row's second segment
+// waits for the stores of its first.  Walk by rows, 30 % new blocks (us):
+//   64 selected, 16 layers of 4x256 q8_0/q4_0 (41 moves)   16: 55  32: 56  64: 62
+//   256 selected, 16 layers of 4x256 q8_0 (177 moves)      16: 309 32: 302 64: 301
+constexpr uint32_t kChainRows = 64;
+constexpr uint32_t kChainRowSel = 4;  // selected blocks per row
 constexpr uint32_t kPlanMaxSel = KVMEM_PLAN_MAX_SEL;    // selected blocks per step (one per thread)
 constexpr uint32_t kPlanMaxSlots = KVMEM_PLAN_MAX_SLOTS;  // pool slots
 constexpr uint16_t kNoMove = 0xffffu;
@@ -2906,9 +2915,8 @@ int kvmem_hip_reselect_device(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist,
     if (injected_fail(ctx, KVMEM_HIP_FAIL_LAUNCH, "reselect_device chain launch")) {
         return KVMEM_HIP_ERR_RUNTIME;
     }
-    // up to kChainRows segments run side by side, one per grid row; more
-    // take turns (a row's next segment waits for its stores)
-    const dim3 cgrid(static_cast<uint32_t>((nvec + 255) / 256), std::min<uint32_t>(kChainRows, max_segs));
+    const dim3 cgrid(static_cast<uint32_t>((nvec + 255) / 256),
+                     std::min<uint32_t>(kChainRows, (max_sel + kChainRowSel - 1) / kChainRowSel));
     move_chain_kernel<uint16_t><<<cgrid, 256, 0, ctx->stream>>>(cp, kNoArgTables);
     if (!hip_ok(ctx, hipGetLastError(), "reselect_device chain launch")) {
         return KVMEM_HIP_ERR_RUNTIME;

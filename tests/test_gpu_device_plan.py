@@ -526,3 +526,46 @@ def test_device_plan_at_and_past_its_limits(oracle, budget, reserve, on_device):
                         assert np.array_equal(pd[2 * layer + which][slots[b]], want), (layer, which, b)
     del k, v
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("budget,runs", [(6, (1, 2)), (24, (1, 8, 9)), (64, (1, 2, 17)), (65, (8, 33))])
+def test_device_plan_shifted_selections(budget, runs):
+    """Selections shifted by 1, 2, ... blocks: chains from one of budget - 1
+    moves to many of one, more segments than the walk has rows, ranks past
+    every cut.  The pool bytes and slots are the host plan's."""
+    announce(f"device plan: budget {budget}, shifts {runs}")
+    lg, tg, hkv, hq, d = 2, 16, 1, 2, 256
+    nb = 4 * budget
+    k, v, q = workloads.scoring_tensors(torch, "cuda", L=lg, B=nb, Tq=1, seed=budget, T=tg, Hkv=hkv, Hq=hq, D=d,
+                                        with_v=True)
+    n_bytes = budget * tg * kv.row_size(kv.TYPE_Q8_0, hkv * d)
+
+    def engine(plan):
+        return host.Engine(n_layers=lg, block_tokens=tg, n_head=hq, n_head_kv=hkv, head_dim=d,
+                           budget_blocks=budget, reserve_blocks=8, device_plan=plan)
+
+    with engine(1) as dev, engine(0) as ref:
+        for eng in (dev, ref):
+            eng.set_device_history(k.data_ptr(), v.data_ptr(), nb, nb * tg)
+        first = budget + 1
+        moved = 0
+        for shift in (0, *runs):
+            first += shift
+            for at in (first, first - shift):  # there and back
+                sel = [0] + list(range(at, at + budget - 1))
+                torch.cuda.synchronize()
+                sd = dev.apply_retrieval(q.data_ptr(), 1, mandatory=sel)
+                sr = ref.apply_retrieval(q.data_ptr(), 1, mandatory=sel)
+                assert sd.pop("device_planned") == 1 and sr.pop("device_planned") == 0
+                assert sd == sr
+                moved += sd["n_moved"]
+                assert dev.block_slots() == ref.block_slots()
+                c = kv.Context(0)
+                for layer in range(lg):
+                    for a, b in zip(dev.pool_layer(layer), ref.pool_layer(layer)):
+                        buf = torch.empty((2, n_bytes), dtype=torch.uint8, device="cuda")
+                        c.d2d_batched([a, b], [buf[0].data_ptr(), buf[1].data_ptr()], [n_bytes, n_bytes])
+                        c.sync()
+                        assert torch.equal(buf[0], buf[1]), (shift, at, layer)
+                c.close()
+        assert moved >= budget
