@@ -588,8 +588,8 @@ KVMEM_HIP_API uint64_t kvmem_hip_debug_fail_left(const kvmem_hip_ctx *ctx);
  * h2d_bytes / d2h_bytes / d2d_bytes: the bytes of kvmem_hip_transfer_get.
  * meank_cos_ms: the mean-K scorer's cosine kernel alone (events attached to
  * its launch), the one kernel of that scorer that streams the key sums;
- * score_ms covers all of its kernels (query, cosine, combine) and the gaps
- * between them.  The per-token scorer is one kernel, timed in score_ms the
+ * score_ms covers both of its kernels (query, cosine) and the gap between
+ * them.  The per-token scorer is one kernel, timed in score_ms the
  * same way. */
 typedef struct kvmem_hip_perf {
     double score_ms;

@@ -481,6 +481,8 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const float m = kc[hh][j][e] * inv;
+                            // one rounding per term: 1.373e-8 rms from 64 bits over 35483
+                            // scores of 31 shapes, 1.374e-8 with a rounded product
                             dot = __builtin_fmaf(q[e], m, dot);
                             nk = __builtin_fmaf(m, m, nk);
                         }
