@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace kvmem_hip {
@@ -199,7 +200,8 @@ __global__ __launch_bounds__(256) void q_accumulate_kernel(const QT *q, const ui
 // WAVES waves of a workgroup (64 channels) each load a run of 32 tokens at
 // once, and the first wave adds all of them in order, its own from registers
 // and the others' from LDS.  Up to 32 tokens take one wave.  128 tokens x 1024
-// f32 channels: 4.4 us; 52.5 with one token in flight at a time.
+// f32 channels: 4.4 us; 52.5 with one token in flight at a time.  (28 tokens of
+// f16: 4.2 us per call; 5.2 while each load's branch also widened its value.)
 constexpr uint32_t kAddRun = 32;
 
 template <typename KT, int WAVES>
@@ -207,6 +209,8 @@ __global__ __launch_bounds__(WAVES * 64) void meank_add_kernel(const uint8_t *k,
                                                                uint32_t head_dim, uint64_t nb0, uint64_t nb1,
                                                                uint64_t nb2, uint32_t tok0, uint32_t n_keep,
                                                                int reset, float *acc, uint32_t *count) {
+    using bits_t = std::conditional_t<sizeof(KT) == 2, uint16_t, uint32_t>;
+    auto widen = [](uint32_t bits) { return static_cast<float>(__builtin_bit_cast(KT, static_cast<bits_t>(bits))); };
     __shared__ float rows[WAVES > 1 ? (WAVES - 1) * kAddRun : 1][64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
@@ -222,20 +226,22 @@ __global__ __launch_bounds__(WAVES * 64) void meank_add_kernel(const uint8_t *k,
     float s = (reset || wave != 0) ? 0.0f : acc[ch];
     for (uint32_t t0 = 0; t0 < n_keep; t0 += WAVES * kAddRun) {
         const uint32_t mine = t0 + wave * kAddRun;
-        float v[kAddRun];
+        // The bits as loaded, each value in a register of its own, widened when
+        // it is added: a conversion (or the packing of two 16-bit values) in
+        // the branch of a load would wait for that load there.
+        uint32_t v[kAddRun];
 #pragma unroll
         for (uint32_t j = 0; j < kAddRun; ++j) {
-            v[j] = 0.0f;
+            v[j] = 0u;
             if (mine + j < n_keep) {
-                v[j] = static_cast<float>(
-                    *reinterpret_cast<const KT *>(base + static_cast<uint64_t>(tok0 + mine + j) * nb2));
+                v[j] = *reinterpret_cast<const bits_t *>(base + static_cast<uint64_t>(tok0 + mine + j) * nb2);
             }
         }
         if (wave == 0) {
 #pragma unroll
             for (uint32_t j = 0; j < kAddRun; ++j) {
                 if (mine + j < n_keep) {
-                    s += v[j];
+                    s += widen(v[j]);
                 }
             }
         }
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(WAVES * 64) void meank_add_kernel(const uint8_t *k,
             if (wave != 0) {
 #pragma unroll
                 for (uint32_t j = 0; j < kAddRun; ++j) {
-                    rows[(wave - 1u) * kAddRun + j][lane] = v[j];
+                    rows[(wave - 1u) * kAddRun + j][lane] = widen(v[j]);
                 }
             }
             __syncthreads();
