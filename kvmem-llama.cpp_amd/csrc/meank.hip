@@ -373,56 +373,99 @@ __device__ inline float row16_sum(float v) {
     return v;
 }
 
-// Cosines and their combination over layers: a workgroup of 8 waves takes
+// Cosines and their combination over layers: a workgroup of WAVES waves takes
 // groups of 4 blocks, every layer of them.  Wave w scores the scored layers w,
-// w + 8, ..., 16 lanes per block: a lane holds D/16 channels of HS heads as
+// w + WAVES, ..., 16 lanes per block: a lane holds D/16 channels of HS heads as
 // float4s (16 KiB per wave with HS = 4 and D = 256), all loaded before the
 // first is reduced, and the next step's loads are issued as soon as the last
-// head is, before the group's layers meet.  The query vectors come from LDS
-// when every layer's fit there (QLDS: loads return in order, so a query load
-// behind key loads would wait for all of them), else from the caches.  The
+// head is, before the group's layers meet.  Ahead of a step's key loads its
+// wave loads the step's query vectors, 4 KiB, and hands them to its lanes
+// through LDS (loads return in order, so a query load behind key loads would
+// wait for all of them: 64 layers x 64 blocks 67 us per call so, 27 as it is).
+// Every layer's in LDS from the start, where they fit, is no faster: 16 layers
+// x 250 blocks 14.0 us per call and 11.6, x 2000 blocks 25.4 and 25.3.  The
 // layers' cosine sums meet in LDS, where one thread per block adds them in
 // layer order (in double): the mean over scored layers of the cosine sum / Hkv,
 // 0 when no layer holds keys of the block.  HBM-bound: every key sum is read
 // once.  16 layers x 2048 blocks of 1024 channels (134 MB): 24.1 us = 5.6 TB/s,
 // where a kernel for the cosines and one for the combination took 34.0 and 5.0
-// with a launch between them.  (Query vectors from the caches: 25.1.)
+// with a launch between them.
 // Workgroups beyond two per CU would start late and run alone: 2100 blocks take
 // 58.3 us per preview with 512 workgroups that go on to the next group, 60.7
 // with one workgroup per group.
+//  - Launches of at most one workgroup per CU with more than 8 layers have 16
+//    waves (the same waves per CU, half the layers one after the other).
+//  - With fewer layers than waves and enough blocks, 2^lw_bits waves take the
+//    layers and the others further groups of 4 blocks.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr uint32_t kCosBlocks = 4;
-constexpr uint32_t kCosWaves = 8;
 constexpr uint32_t kCosGroups = 512;      // workgroups of a launch, at most: two per CU
-constexpr uint32_t kCosLds = 79 * 1024;   // LDS that leaves room for two workgroups per CU
 extern __shared__ float4 cos_lds[];
 
-// Dynamic LDS: the layers' cosine sums of two groups, then (QLDS) the query
-// vectors and their norms.
-static size_t cos_lds_bytes(uint32_t L, uint32_t Hkv, uint32_t D, bool q_lds) {
-    const size_t term = sizeof(double) * 2u * kCosBlocks * L;
-    return term + (q_lds ? sizeof(float) * static_cast<size_t>(L) * Hkv * (D + 1u) : 0u);
+// The launch shape of a call: waves of a workgroup, log2 of those that take
+// layers side by side, workgroups, heads of a step, and the dynamic LDS: the
+// layers' cosine sums of two turns, then each wave's query vectors of a step.
+struct CosShape {
+    uint32_t waves = 8, lw_bits = 3, grid = 0, heads = 4, lds = 0;
+};
+
+static CosShape cos_shape(uint32_t n_scored, uint32_t B, uint32_t Hkv, uint32_t D) {
+    CosShape s;
+    // steps of four heads, or of two where four would load heads twice
+    if (Hkv % 4u != 0 && (Hkv + 1u) / 2u * 2u < (Hkv + 3u) / 4u * 4u) {
+        s.heads = 2;
+    }
+    uint32_t blocks = kCosBlocks;  // of a workgroup's turn
+    if (n_scored > 8u && B <= kCosGroups / 2u * blocks) {
+        s.waves = 16;
+        s.lw_bits = 4;
+    }
+    while (s.lw_bits > 0u && n_scored <= 1u << (s.lw_bits - 1u) && B >= kCosGroups * 2u * blocks) {
+        --s.lw_bits;
+        blocks *= 2u;
+    }
+    s.grid = std::min((B + blocks - 1u) / blocks, kCosGroups);
+    s.lds = static_cast<uint32_t>(sizeof(double) * 2u * blocks * n_scored + sizeof(float) * s.waves * s.heads * D);
+    return s;
 }
 
-template <int D, int HS, bool QLDS>
-__global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void meank_score_kernel(
-    const float *k_sum, const uint32_t *mean_tokens, const float *qv, const float *nq, ScoredLayers scored, uint32_t L,
-    uint32_t B, uint32_t cap, uint32_t Hkv, float *scores) {
-    constexpr int P4 = D / 64;  // float4s per lane per head
-    __shared__ uint32_t has_keys[2][kCosWaves][kCosBlocks];
-    double *term = reinterpret_cast<double *>(cos_lds);  // [2][kCosBlocks][L]
-    f32x4_t *q_lds = reinterpret_cast<f32x4_t *>(cos_lds) + kCosBlocks * L;
+template <int D, int HS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void meank_score_kernel(
+    const float *k_sum, const uint32_t *mean_tokens, const float *qv, const float *nq, ScoredLayers scored,
+    uint32_t lw_bits, uint32_t L, uint32_t B, uint32_t cap, uint32_t Hkv, float *scores) {
+    constexpr int P4 = D / 64;             // float4s per lane per head
+    constexpr int NQ = HS * (D / 4) / 64;  // float4s per lane of a step's query vectors
+    __shared__ uint32_t has_keys[2][WAVES][kCosBlocks];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t sub = lane & 15u;
     const uint32_t lb = lane >> 4;
+    const uint32_t lw = 1u << lw_bits;
+    const uint32_t first = wave & (lw - 1u);                // the wave's first scored layer
+    const uint32_t in_turn = (wave >> lw_bits) * kCosBlocks + lb;  // the lane's block among the turn's
+    const uint32_t per_turn = (WAVES >> lw_bits) * kCosBlocks;
     const uint32_t row4 = Hkv * (D / 4);  // float4s of a key-sum row
-    const uint32_t n_groups = (B + kCosBlocks - 1u) / kCosBlocks;
+    const uint32_t n_groups = (B + per_turn - 1u) / per_turn;
+    double *term = reinterpret_cast<double *>(cos_lds);  // [2][per_turn][scored.n]
+    f32x4_t *q_lds = reinterpret_cast<f32x4_t *>(term + 2u * per_turn * scored.n) + wave * HS * (D / 4);
 
     // a step: HS heads of one scored layer, loaded together
     f32x4_t kc[HS][P4];
-    auto block_of = [&](uint32_t g) { return min(g * kCosBlocks + lb, B - 1u); };  // past the end: not stored
+    float qn[HS];  // query norms
+    auto block_of = [&](uint32_t g) { return min(g * per_turn + in_turn, B - 1u); };  // past the end: not stored
     auto load_step = [&](uint32_t g, uint32_t l, uint32_t h0) {
+        f32x4_t q[NQ];
+#pragma unroll
+        for (int hh = 0; hh < HS; ++hh) {
+            qn[hh] = nq[l * Hkv + min(h0 + hh, Hkv - 1u)];
+        }
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+            const uint32_t at = j * 64 + lane;
+            const uint32_t h = min(h0 + at / (D / 4), Hkv - 1u);
+            q[j] = reinterpret_cast<const f32x4_t *>(qv)[l * row4 + h * (D / 4) + at % (D / 4)];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // ahead of the keys
         const f32x4_t *row = reinterpret_cast<const f32x4_t *>(k_sum) +
                              (static_cast<uint64_t>(l) * cap + block_of(g)) * row4 + sub;
 #pragma unroll
@@ -435,33 +478,26 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
             }
         }
         __builtin_amdgcn_sched_barrier(0);  // all of them before the first use
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {  // (the wave has read the last step's)
+            q_lds[j * 64 + lane] = q[j];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
     auto load_tokens = [&](uint32_t g, uint32_t l) { return mean_tokens[static_cast<uint64_t>(l) * cap + block_of(g)]; };
     uint32_t g = blockIdx.x;  // (the grid has at most n_groups workgroups)
     uint32_t mt = 0;          // tokens of the step's layer in the lane's block
-    if (wave < scored.n) {
-        mt = load_tokens(g, scored.l[wave]);
-        load_step(g, scored.l[wave], 0u);
-    }
-    const float *q_norm = nq;
-    if constexpr (QLDS) {
-        const f32x4_t *src = reinterpret_cast<const f32x4_t *>(qv);
-        for (uint32_t t = threadIdx.x; t < L * row4; t += kCosWaves * 64u) {
-            q_lds[t] = src[t];
-        }
-        float *norms = reinterpret_cast<float *>(q_lds + L * row4);
-        for (uint32_t t = threadIdx.x; t < L * Hkv; t += kCosWaves * 64u) {
-            norms[t] = nq[t];
-        }
-        __syncthreads();
-        q_norm = norms;
+    if (first < scored.n) {
+        mt = load_tokens(g, scored.l[first]);
+        load_step(g, scored.l[first], 0u);
     }
     uint32_t turn = 0;
     for (; g < n_groups; g += gridDim.x, turn ^= 1u) {
         uint32_t has = 0;
-        for (uint32_t i = wave; i < scored.n; i += kCosWaves) {
+        for (uint32_t i = first; i < scored.n; i += lw) {
             const uint32_t l = scored.l[i];
-            const f32x4_t *qs = (QLDS ? q_lds : reinterpret_cast<const f32x4_t *>(qv)) + l * row4 + sub;
             const float inv = mt ? 1.0f / static_cast<float>(mt) : 0.0f;
             double layer = 0.0;
             for (uint32_t h0 = 0; h0 < Hkv; h0 += HS) {
@@ -479,11 +515,11 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
                 }
 #pragma unroll
                 for (int hh = 0; hh < HS; ++hh) {
-                    const uint32_t h = min(h0 + hh, Hkv - 1u);
+                    const f32x4_t *qs = q_lds + hh * (D / 4) + sub;
                     float dot = 0.0f, nk = 0.0f;
 #pragma unroll
                     for (int j = 0; j < P4; ++j) {
-                        const f32x4_t q = qs[h * (D / 4) + j * 16];
+                        const f32x4_t q = qs[j * 16];
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const float m = kc[hh][j][e] * inv;
@@ -496,25 +532,25 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
                     dot = row16_sum(dot);
                     nk = row16_sum(nk);
                     if (h0 + hh < Hkv) {
-                        layer += static_cast<double>(dot / (q_norm[l * Hkv + h] * sqrtf(nk) + 1e-6f));
+                        layer += static_cast<double>(dot / (qn[hh] * sqrtf(nk) + 1e-6f));
                     }
                 }
             }
             has |= mt;
             // the wave's next step: its next layer, or its first of the next group
-            const bool more = i + kCosWaves < scored.n;
+            const bool more = i + lw < scored.n;
             const uint32_t gn = more ? g : g + gridDim.x;
             if (gn < n_groups) {
-                const uint32_t ln = scored.l[more ? i + kCosWaves : wave];
+                const uint32_t ln = scored.l[more ? i + lw : first];
                 mt = load_tokens(gn, ln);
                 load_step(gn, ln, 0u);
             }
             if (sub == 0u) {
-                term[(turn * kCosBlocks + lb) * L + i] = layer / static_cast<double>(Hkv);
+                term[(turn * per_turn + in_turn) * scored.n + i] = layer / static_cast<double>(Hkv);
             }
         }
         if (scored.n != L) {  // the layers without query rows count here too
-            for (uint32_t u = wave; u < L; u += kCosWaves) {
+            for (uint32_t u = first; u < L; u += lw) {
                 has |= load_tokens(g, u);
             }
         }
@@ -523,16 +559,16 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
         }
         __syncthreads();  // (the next group's terms go to the other half)
         const uint32_t t = threadIdx.x;
-        const uint32_t b = g * kCosBlocks + t;
-        if (t < kCosBlocks && b < B) {
+        const uint32_t b = g * per_turn + t;
+        if (t < per_turn && b < B) {
+            const uint32_t w0 = (t / kCosBlocks) << lw_bits;
             uint32_t any = 0;
-#pragma unroll
-            for (uint32_t w = 0; w < kCosWaves; ++w) {
-                any |= has_keys[turn][w][t];
+            for (uint32_t w = 0; w < lw; ++w) {
+                any |= has_keys[turn][w0 + w][t % kCosBlocks];
             }
             double acc = 0.0;
             for (uint32_t u = 0; u < scored.n; ++u) {
-                acc += term[(turn * kCosBlocks + t) * L + u];
+                acc += term[(turn * per_turn + t) * scored.n + u];
             }
             scores[b] = static_cast<float>((any && scored.n) ? acc / scored.n : 0.0);
         }
@@ -540,15 +576,14 @@ __global__ __launch_bounds__(kCosWaves * 64) __attribute__((amdgpu_waves_per_eu(
 }
 
 using MeankScoreKernel = void (*)(const float *, const uint32_t *, const float *, const float *, ScoredLayers, uint32_t,
-                                  uint32_t, uint32_t, uint32_t, float *);
+                                  uint32_t, uint32_t, uint32_t, uint32_t, float *);
 
 template <int D>
-static MeankScoreKernel meank_score_of(uint32_t Hkv, bool q_lds) {
-    // steps of four heads, or of two where four would load heads twice
-    if (Hkv % 4u != 0 && (Hkv + 1u) / 2u * 2u < (Hkv + 3u) / 4u * 4u) {
-        return q_lds ? meank_score_kernel<D, 2, true> : meank_score_kernel<D, 2, false>;
+static MeankScoreKernel meank_score_of(const CosShape &s) {
+    if (s.heads == 2u) {
+        return s.waves == 16u ? meank_score_kernel<D, 2, 16> : meank_score_kernel<D, 2, 8>;
     }
-    return q_lds ? meank_score_kernel<D, 4, true> : meank_score_kernel<D, 4, false>;
+    return s.waves == 16u ? meank_score_kernel<D, 4, 16> : meank_score_kernel<D, 4, 8>;
 }
 
 size_t meank_scratch_bytes(uint32_t L, uint32_t Hkv, uint32_t B, uint32_t D) {
@@ -557,7 +592,7 @@ size_t meank_scratch_bytes(uint32_t L, uint32_t Hkv, uint32_t B, uint32_t D) {
 }
 
 bool load_meank_kernels() {
-    return load_kernel_object(&meank_score_kernel<256, 4, true>);
+    return load_kernel_object(&meank_score_kernel<256, 4, 8>);
 }
 
 }  // namespace kvmem_hip
@@ -803,15 +838,13 @@ int kvmem_hip_score_meank(kvmem_hip_ctx *ctx, const kvmem_hip_meank_args *a) {
     perf_begin(ctx, kPerfScore);
     const uint32_t lh = L * a->n_head_kv;
     meank_query_kernel<<<lh, D, 0, ctx->stream>>>(a->q_sum, invq, L, a->n_head, a->n_head_kv, D, qv, nq);
-    const uint32_t grid = std::min((B + kCosBlocks - 1) / kCosBlocks, kCosGroups);
+    const CosShape shape = cos_shape(scored.n, B, a->n_head_kv, D);
     {
         // the kernel which streams the key sums, also timed alone
         PerfLaunchScope timed(ctx, kPerfMeankCos);
-        const bool q_lds = cos_lds_bytes(L, a->n_head_kv, D, true) <= kCosLds;
-        ctx_launch(ctx, D == 256 ? meank_score_of<256>(a->n_head_kv, q_lds) : meank_score_of<128>(a->n_head_kv, q_lds),
-                   dim3(grid), dim3(kCosWaves * 64u),
-                   static_cast<uint32_t>(cos_lds_bytes(L, a->n_head_kv, D, q_lds)), a->k_sum, a->mean_tokens, qv, nq,
-                   scored, L, B, cap, a->n_head_kv, a->scores);
+        ctx_launch(ctx, D == 256 ? meank_score_of<256>(shape) : meank_score_of<128>(shape), dim3(shape.grid),
+                   dim3(shape.waves * 64u), shape.lds, a->k_sum, a->mean_tokens, qv, nq, scored, shape.lw_bits, L, B, cap,
+                   a->n_head_kv, a->scores);
         if (hip_ok(ctx, hipGetLastError(), "score_meank launch")) {
             timed.ok();
         } else {

@@ -469,3 +469,32 @@ def test_meank_scores_step_edges(ctx, L_, nb, Hkv, Dh, g):
     err = float((scores[:nb].double() - want).abs().max())
     assert err <= 3 * (Dh / 16 + 5 + g) * 2.0 ** -24, err
     assert float(scores[nb]) == -9.0
+
+
+@pytest.mark.parametrize("L_,nb,Hkv,Dh,g", [
+    (1, 16390, 2, 128, 2),   # one layer: every wave takes blocks of its own, the last turn short
+    (2, 8203, 1, 128, 1),    # one scored layer of two, the other only counts keys
+    (3, 4101, 5, 128, 3),    # two scored layers on four waves, steps of two heads
+    (14, 1024, 3, 128, 2),   # 9 scored layers on 16 waves, a workgroup per CU
+    (14, 1025, 4, 256, 1),   # and on 8 waves, a workgroup more
+    (100, 19, 4, 256, 6),    # several layers to each of 16 waves
+    (49, 1027, 2, 256, 2),   # and of 8
+])
+def test_meank_scores_launch_shapes(ctx, L_, nb, Hkv, Dh, g):
+    """The same against 64 bits over the launch shapes: waves that share
+    layers, waves that share blocks, 8 and 16 waves."""
+    test_meank_scores_step_edges(ctx, L_, nb, Hkv, Dh, g)
+
+
+@pytest.mark.parametrize("nb", [7, 9000])
+def test_meank_scores_without_query_rows(ctx, nb):
+    """No layer has query rows: every score is zero."""
+    announce(f"mean-K scores without query rows: 3 layers x {nb} blocks")
+    ks = torch.ones((3, nb, 256), dtype=torch.float32, device="cuda")
+    mt = torch.full((3, nb), 4, dtype=torch.int32, device="cuda")
+    q_sum = torch.ones((3, 256), dtype=torch.float32, device="cuda")
+    scores = torch.full((nb + 1,), -9.0, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    ctx.score_meank(q_sum.data_ptr(), [0, 0, 0], ks.data_ptr(), mt.data_ptr(), 3, nb, 2, 2, 128, scores.data_ptr())
+    ctx.sync()
+    assert not scores[:nb].any() and float(scores[nb]) == -9.0
