@@ -16,7 +16,9 @@
 // (Scores of one call share their sign and most of their exponent.  A pass
 // over those bits puts nearly every key into one histogram word, where the
 // LDS atomics of a wave queue up.  2048 scores: 8.3 us, 10.0 with passes from
-// the top bit and four barriers each; 8192 scores: 12.7 and 21.0.)
+// the top bit and four barriers each; 8192 scores: 12.7 and 21.0.  Mean cosines
+// have both signs and gain nothing: the bit is found while the keys are made,
+// and the streamed kernel looks at 1024 scores before it spends a pass on it.)
 // Winners are the keys at or above that threshold; they and the forced ids are
 // compacted in ascending id order with a workgroup prefix sum, which is the
 // window order of KvMemStore::pick_topk_ungrouped (kvmem_store.cpp:618-622).
@@ -110,40 +112,44 @@ struct RadixShared {
     uint32_t alone;
 };
 
-// The key of rank `need` (from the largest; need > 0, at most the number of
-// candidates) among key_of(0 .. n), 0 = no candidate, on the bits of `mask`: a
-// candidate is of that rank or better when its key on those bits is >= the
-// value returned.  Keys are unique, so once the digit holding the rank has a
-// single key the digits decided so far order every other key against it, and
-// the later passes are skipped.  Called by the whole workgroup.
-template <class KeyOf>
-__device__ inline uint64_t radix_threshold(uint32_t n, uint32_t need, bool tie_lower, const KeyOf &key_of,
-                                           RadixShared &sh, uint64_t &mask) {
+// One wave's share of the OR of the workgroup's score words and of their
+// complements, and cleared digit counts; score_bits() reads both after a
+// barrier.
+__device__ inline void put_score_bits(uint32_t ones, uint32_t zeros, RadixShared &sh) {
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    uint32_t ones = 0u, zeros = 0u;
-    for (uint32_t i = tid; i < n; i += kTopkThreads) {
-        const uint64_t k = key_of(i);
-        if (k != 0ull) {
-            ones |= static_cast<uint32_t>(k >> 32);
-            zeros |= ~static_cast<uint32_t>(k >> 32);
-        }
-    }
     ones = wave_or(ones);
     zeros = wave_or(zeros);
-    if (lane == 0u) {
+    if ((tid & 63u) == 0u) {
         sh.ones[tid >> 6] = ones;
         sh.zeros[tid >> 6] = zeros;
     }
     if (tid < 256u) {
         sh.hist[tid] = 0u;
     }
-    __syncthreads();
+}
+__device__ inline void score_bits(const RadixShared &sh, uint32_t &ones, uint32_t &zeros) {
+    ones = zeros = 0u;
 #pragma unroll
     for (int w = 0; w < kTopkWaves; ++w) {
         ones |= sh.ones[w];
         zeros |= sh.zeros[w];
     }
+}
+
+// The key of rank `need` (from the largest; need > 0, at most the number of
+// candidates) among key_of(0 .. n), 0 = no candidate, on the bits of `mask`: a
+// candidate is of that rank or better when its key on those bits is >= the
+// value returned.  Keys are unique, so once the digit holding the rank has a
+// single key the digits decided so far order every other key against it, and
+// the later passes are skipped.  `ones` and `zeros` are the OR of the score
+// words and of their complements over the candidates and perhaps others (a
+// bit that is in only one of them is the same in every candidate).  Called by
+// the whole workgroup, with put_score_bits() and a barrier before.
+template <class KeyOf>
+__device__ inline uint64_t radix_threshold(uint32_t n, uint32_t need, bool tie_lower, const KeyOf &key_of,
+                                           RadixShared &sh, uint32_t ones, uint32_t zeros, uint64_t &mask) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u;
     // key bits still open: from the scores' highest differing bit down
     const uint32_t differ = ones & zeros;
     const uint32_t id_bits = n > 1u ? 32u - static_cast<uint32_t>(__clz(static_cast<int>(n - 1u))) : 0u;
@@ -232,9 +238,14 @@ __global__ __launch_bounds__(kTopkThreads) void topk_kernel(const float *scores,
     const uint32_t tid = threadIdx.x;
     const bool tl = tie_lower != 0;
 
+    uint32_t ones = 0u, zeros = 0u;  // over forced ids too: the passes may start a bit high
     for (uint32_t i = tid; i < n; i += kTopkThreads) {
-        keys[i] = rank_key(scores[i], i, tl);
+        const uint64_t k = rank_key(scores[i], i, tl);
+        keys[i] = k;
+        ones |= static_cast<uint32_t>(k >> 32);
+        zeros |= ~static_cast<uint32_t>(k >> 32);
     }
+    put_score_bits(ones, zeros, radix);
     for (uint32_t w = tid; w < (n + 31u) / 32u; w += kTopkThreads) {
         forced_bits[w] = 0u;
     }
@@ -246,9 +257,10 @@ __global__ __launch_bounds__(kTopkThreads) void topk_kernel(const float *scores,
     }
     __syncthreads();
 
+    score_bits(radix, ones, zeros);
     uint64_t mask = 0ull;
     const uint64_t threshold =
-        need > 0u ? radix_threshold(n, need, tl, [&](uint32_t i) { return keys[i]; }, radix, mask) : 0ull;
+        need > 0u ? radix_threshold(n, need, tl, [&](uint32_t i) { return keys[i]; }, radix, ones, zeros, mask) : 0ull;
 
     // ---- ordered compaction: thread t owns ids [t*seg, (t+1)*seg)
     const uint32_t seg = (n + kTopkThreads - 1) / kTopkThreads;
@@ -330,8 +342,35 @@ __global__ __launch_bounds__(kTopkThreads) void topk_stream_kernel(
     auto is_forced = [&](uint32_t i) -> bool { return (forced_bits[i >> 5] >> (i & 31u)) & 1u; };
     auto key_of = [&](uint32_t i) -> uint64_t { return is_forced(i) ? 0ull : rank_key(scores[i], i, tl); };
 
+    // Where the first scores (one per thread) differ in their top byte, the
+    // passes start there, at once; else a pass over the rest finds the bit.
+    uint32_t ones = 0u, zeros = 0u;
+    auto add_bits = [&](uint32_t i) {
+        const uint32_t u = static_cast<uint32_t>(rank_key(scores[i], i, tl) >> 32);
+        ones |= u;
+        zeros |= ~u;
+    };
+    add_bits(tid);  // (n > kTopkThreads)
+    put_score_bits(ones, zeros, radix);
+    __syncthreads();
+    score_bits(radix, ones, zeros);
+    if (((ones & zeros) >> 24) != 0u) {
+        ones = zeros = ~0u;
+    } else {
+        for (uint32_t i = tid + kTopkThreads; i < n; i += 8u * kTopkThreads) {
+#pragma unroll
+            for (uint32_t j = 0; j < 8u; ++j) {  // (past the end: the last score again)
+                add_bits(min(i + j * kTopkThreads, n - 1u));
+            }
+        }
+        __syncthreads();  // the words are read before they are written again
+        put_score_bits(ones, zeros, radix);
+        __syncthreads();
+        score_bits(radix, ones, zeros);
+    }
+
     uint64_t mask = 0ull;
-    const uint64_t threshold = need > 0u ? radix_threshold(n, need, tl, key_of, radix, mask) : 0ull;
+    const uint64_t threshold = need > 0u ? radix_threshold(n, need, tl, key_of, radix, ones, zeros, mask) : 0ull;
     auto chosen = [&](uint32_t i) -> bool {
         if (is_forced(i)) {
             return true;

@@ -203,3 +203,20 @@ def test_topk_radix_windows(ctx, oracle, kind, n, need, tie_lower):
     torch.cuda.synchronize()
     got = ctx.topk(d.data_ptr(), n, need, forced=[0], tie_lower_index=tie_lower)
     assert got == oracle.pick_topk(s.astype(np.float64), need + 1, sink=1, tie_lower_index=tie_lower)
+
+
+@pytest.mark.parametrize("n", [1025, 16384, 16385, 20000])
+@pytest.mark.parametrize("late", [-1.0, 6.0000005, 1e30])
+@pytest.mark.parametrize("forced_score", [6.0, -3e38])
+def test_topk_radix_start(ctx, oracle, n, late, forced_score):
+    """Scores that differ only past the first 1024 of them, by a sign, one bit
+    or an exponent, beside a forced id whose own score is far from the rest."""
+    announce(f"radix start: n={n} late={late} forced score {forced_score}")
+    s = np.full(n, 6.0, np.float32)
+    s[0] = forced_score
+    s[1024::7] = late
+    for need in (1, n // 2):
+        d = dev(s)
+        torch.cuda.synchronize()
+        got = ctx.topk(d.data_ptr(), n, need, forced=[0])
+        assert got == oracle.pick_topk(s.astype(np.float64), need + 1, sink=1)
