@@ -688,8 +688,23 @@ int score_setup(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist, const kvmem_h
         // consecutive on one XCD, and chunks of at most 64 blocks keep them
         // close enough together for a tile to come from that XCD's L2 (16 x
         // 8192 blocks, 512-token query: 65.3 ms; 67.6 with 16 blocks per
-        // chunk, 65.7 with 256).
-        p.blocks_per_chunk = std::min(p.blocks_per_chunk, 64u);
+        // chunk, 65.7 with 256).  Up to there the chunk of the least cost: a
+        // workgroup's blocks and its start-up, which is worth about 128 keys,
+        // by the rounds of workgroups, half as if they ran in step (a short
+        // last round leaves the chip idle) and half as if they did not.  16
+        // layers x 50 blocks, 384-token query: 343 us (13 blocks per chunk; 394
+        // in one round of 50, 371 in 3.75 of 10); 2 x 1454, 512-token query:
+        // 1136 us (1256 with 64 blocks per chunk, 1225 with 35).
+        const uint32_t chip = full / shape.wr;
+        double best = 0.0;
+        for (uint32_t bpc = std::min(B, 64u); bpc > 0; --bpc) {
+            const double rounds = static_cast<double>(pairs) * p.RG * ((B + bpc - 1) / bpc) / chip;
+            const double cost = (rounds + std::ceil(rounds)) * (bpc + 128.0 / p.T);
+            if (best == 0.0 || cost < best) {
+                best = cost;
+                p.blocks_per_chunk = bpc;
+            }
+        }
     }
     p.n_chunks = (B + p.blocks_per_chunk - 1) / p.blocks_per_chunk;
     p.xcd_major = (pairs % 8u) == 0;
