@@ -158,7 +158,8 @@ struct BlockSource {
     uint32_t n_rot;                   // RoPE rotary dims (0 = none)
     uint32_t hadamard;                // Hadamard width (0 = none)
     float hscale;                     // 1 / sqrtf(hadamard)
-    uint32_t layer_group;             // layers per workgroup chunk index (RoPE'd K: 4; else 1)
+    uint32_t layer_group;             // consecutive layers of a workgroup: 4 for RoPE'd K, else 1;
+                                      // 64-per-lane kernels: all, or a part (launch_block_job)
     uint32_t lw_bits;                 // 64-per-lane kernels: log2 of a workgroup's layer waves
     __device__ void bind(const ArgTables &t) {
         const uint8_t *b = table_base(tables, t);
@@ -1001,9 +1002,9 @@ constexpr uint32_t kX64Wave = 64u * kX64Lane;   // LDS bytes of one wave
 constexpr uint32_t kX64FullGrid = 1024;  // workgroups: four per CU
 constexpr uint32_t kX64Groups = 128; // groups of 32 elements in a unit
 
-// cos/sin table of rotary pairs (n_rot = 2 * half, half 64 or 128) in
-// 16-byte units of two pairs (c_j, s_j, c_j+1, s_j+1).  A lane reads P = 64
-// consecutive pairs; a row holds half / P runs of P/2 units, each followed
+// cos/sin table of rotary pairs (n_rot = 2 * half; half 32, 64 or 128) in
+// 16-byte units of two pairs (c_j, s_j, c_j+1, s_j+1).  A lane reads P
+// consecutive pairs, 64 (32 where half is 32); a row holds half / P runs of P/2 units, each followed
 // by one unused unit, so that the rows and runs one wave-wide read touches
 // fall on distinct banks.
 struct X64Tab {
@@ -1241,9 +1242,8 @@ __device__ inline void x64_quant_lane(const float x[64], float f, float sf, uint
 
 // Workgroup `c` of a block source on this path: chunk `sub` of one block for
 // layer_group consecutive layers.  LW = 2^lw_bits waves take layers side by
-// side, the w-th the w-th, (w + LW)-th, ...: four, or 2 or 1 where the job has
-// fewer layers; then the chunk has 2 or 4 units, for the other waves (50 blocks
-// of one layer: 17.3 us, 29.1 with three waves idle).
+// side, the w-th the w-th, (w + LW)-th, ...: four, or in a large job of few
+// layers 2 or 1; then the chunk has 2 or 4 units, for the other waves.
 template <int TYPE, bool ROPE64>
 __device__ inline void x64_unit_layers(const BlockSource &s, uint32_t c, uint8_t *lds, uint8_t *tab) {
     constexpr int GB = Fmt<TYPE>::GB;
@@ -1705,6 +1705,14 @@ static uint32_t item_pos0(const kvmem_hip_pool *pool, const uint32_t *block_ids,
     return block_ids[i] * block_tokens;
 }
 
+// Gives a workgroup of the 64-per-lane kernels 2^lw_bits layer waves, and a
+// unit for each group of that many.
+static void x64_units(BlockSource &s, uint32_t lw_bits) {
+    s.lw_bits = lw_bits;
+    s.chunk_groups = kX64Groups << (2u - lw_bits);
+    s.chunks_per_op = (s.block_tokens * s.gpr + s.chunk_groups - 1) / s.chunk_groups;
+}
+
 // Source of one kind (K or V) of a block job over the job's tables, its
 // items starting at `first_item`.
 static BlockSource make_block_source(int type, const uint8_t *base, uint64_t block_stride,
@@ -1729,10 +1737,8 @@ static BlockSource make_block_source(int type, const uint8_t *base, uint64_t blo
     s.n_rot = is_k ? xp.n_rot : 0u;
     s.hadamard = is_k ? xp.had_k : xp.had_v;
     s.hscale = is_k ? xp.hscale_k : xp.hscale_v;
-    if (xp.lane64) {  // units of 128 groups, every layer (launch_block_job may split them)
-        s.lw_bits = n_layers >= 4u ? 2u : n_layers >= 2u ? 1u : 0u;
-        s.chunk_groups = kX64Groups << (2u - s.lw_bits);
-        s.chunks_per_op = (block_tokens * s.gpr + s.chunk_groups - 1) / s.chunk_groups;
+    if (xp.lane64) {  // a unit of 128 groups, every layer (launch_block_job fits them to the job)
+        x64_units(s, 2u);
         s.layer_group = n_layers;
     } else {
         s.layer_group = (xp.on && s.n_rot) ? kRopeLayerGroup : 1u;
@@ -1808,15 +1814,36 @@ static int launch_block_job(kvmem_hip_ctx *ctx, int type_k, const BlockSource &k
     BlockSource sk = k, sv_copy = v ? *v : BlockSource{};
     const BlockSource *sv = v ? &sv_copy : nullptr;
     if (xp.lane64) {
+        auto grid = [&]() { return block_job_chunks(sk, n_items) + (sv ? block_job_chunks(*sv, n_items) : 0); };
+        // With one or two layers, further units for the waves without a layer
+        // once the job has more workgroups than the chip holds (1 layer of
+        // 1024 elements, RoPE 64 and attn_rot, q8_0: 64 blocks 31.8 us without,
+        // 15.4 with four units per workgroup; 16 blocks, 1024 workgroups, 11.3
+        // without and 11.5 with two).  Three layers on two waves leave as many
+        // idle as on four; a job past twice the chip still gains from the fewer
+        // workgroups (64 blocks, attn_rot: 40.5 and 38.2), less than the larger
+        // tables of 256 rotary dims cost it (45.3 and 48.2).
+        auto pack = [&]() {
+            if (sk.lw_bits == 0u) {
+                return false;
+            }
+            return sk.n_layers <= 1u << (sk.lw_bits - 1u)
+                       ? grid() > kX64FullGrid
+                       : sk.n_layers == 3u && sk.lw_bits == 2u && sk.n_rot <= 128u && grid() >= 2u * kX64FullGrid;
+        };
+        while (pack()) {
+            x64_units(sk, sk.lw_bits - 1u);
+            x64_units(sv_copy, sk.lw_bits);
+        }
         // A workgroup takes every layer of a unit (one cos/sin table), a wave
-        // one after the other.  Below four workgroups per CU that leaves the
-        // chip empty, and the layers are split over more workgroups (16
-        // layers, RoPE 256 and attn_rot: one block 12.3 us, 35.7 unsplit; four
-        // 16.0 and 37.3).  Splitting also where 1536 workgroups fill the
-        // chip, for an even end, costs more tables than it gains (24 blocks:
-        // 63.9 us, 67.3 split).
-        while (sk.layer_group > 4u &&
-               block_job_chunks(sk, n_items) + (sv ? block_job_chunks(*sv, n_items) : 0) < kX64FullGrid) {
+        // one after the other, which leaves a job of few units most of the chip
+        // empty: there the layers are split over more workgroups (16 layers,
+        // RoPE 256 and attn_rot: one block 12.3 us, 35.7 unsplit).  Halves that
+        // no longer fit the chip at once still pay where they are long (8
+        // layers, attn_rot, by workgroups unsplit: 576 17.6 and 19.7, 704 20.2
+        // and 20.5, 832 23.1 and 22.1; 24 layers: 832 55.0 and 58.8, 960 61.4
+        // and 62.1).
+        while (sk.layer_group > 4u && grid() * sk.layer_group <= uint64_t{kX64FullGrid} * (sk.layer_group - 2u)) {
             sk.layer_group = ((sk.layer_group + 1u) / 2u + 3u) / 4u * 4u;
             sv_copy.layer_group = sk.layer_group;
         }

@@ -240,3 +240,22 @@ def test_transform_layer_splits(ctx, oracle, L, D, hkv, n_rot, hk, tk, tv, last)
     announce(f"{L} layers, head_dim {D} x {hkv}, n_rot {n_rot}, Hadamard {hk}, K={tk} V={tv}, last {last}")
     run_case(ctx, oracle, L=L, B=3, Hkv=hkv, D=D, type_k=tk, type_v=tv, n_rot=n_rot, had_k=hk, had_v=64,
              ids=[2, 0], slots=[3, 1], n_slots=4, last=last, pos0=[1 << 18, 77], seed=L + D + last)
+
+
+@pytest.mark.parametrize("L,B,D,hkv,n_rot,hk,tk,tv,last", [
+    (1, 65, 128, 2, 64, 128, kv.TYPE_Q8_0, kv.TYPE_Q4_0, 3),    # two units per workgroup
+    (1, 130, 256, 1, 0, 256, kv.TYPE_Q5_0, kv.TYPE_Q8_0, 77),   # four
+    (1, 260, 64, 2, 64, 64, kv.TYPE_Q8_0, kv.TYPE_Q8_0, 33),    # four, 128-element rows
+    (2, 70, 128, 2, 128, 0, kv.TYPE_F16, kv.TYPE_F16, 9),       # two layers beside two units
+    (3, 70, 64, 4, 64, 64, kv.TYPE_Q4_0, kv.TYPE_Q5_0, 1),      # three layers: a unit per workgroup
+    (6, 64, 128, 2, 64, 128, kv.TYPE_Q8_0, kv.TYPE_Q8_0, 65),   # six layers to a workgroup of a full chip
+])
+def test_transform_full_chip(ctx, oracle, L, B, D, hkv, n_rot, hk, tk, tv, last):
+    """Jobs of more units than the chip holds workgroups: with one or two
+    layers a workgroup of the 64-elements-per-lane kernel takes several, those
+    of the partial last block without rows among them."""
+    announce(f"{L} layers x {B} blocks, head_dim {D} x {hkv}, n_rot {n_rot}, Hadamard {hk}, K={tk} V={tv}")
+    rng = np.random.default_rng(B)
+    run_case(ctx, oracle, L=L, B=B, Hkv=hkv, D=D, type_k=tk, type_v=tv, n_rot=n_rot, had_k=hk,
+             had_v=64 if hk else 0, ids=rng.permutation(B).tolist(), slots=rng.permutation(B + 1)[:B].tolist(),
+             n_slots=B + 1, last=last, seed=B + L)
