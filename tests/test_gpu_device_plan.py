@@ -226,8 +226,8 @@ def test_perf_stage_mask_and_after_score_span():
 
 
 XF_CASES = [
-    # (n_rot, type_k, type_v): RoPE 256 + attn_rot on the 64-elements-per-lane kernel,
-    # RoPE 64 + attn_rot on the 8-per-lane kernel, attn_rot alone
+    # (n_rot, type_k, type_v): RoPE 256 + attn_rot, RoPE 64 + attn_rot and attn_rot
+    # alone, all on the 64-elements-per-lane kernel
     (256, kv.TYPE_Q8_0, kv.TYPE_Q4_0),
     (64, kv.TYPE_Q5_0, kv.TYPE_Q5_0),
     (0, kv.TYPE_Q8_0, kv.TYPE_Q8_0),
@@ -569,3 +569,13 @@ def test_device_plan_shifted_selections(budget, runs):
                         assert torch.equal(buf[0], buf[1]), (shift, at, layer)
                 c.close()
         assert moved >= budget
+
+
+@pytest.mark.parametrize("n_rot,tk,tv", [(48, kv.TYPE_Q8_0, kv.TYPE_Q4_0), (32, kv.TYPE_Q5_0, kv.TYPE_Q5_0),
+                                         (96, kv.TYPE_F16, kv.TYPE_Q8_0)],
+                         ids=["rope48_q8q4", "rope32_q5q5", "rope96_f16q8"])
+def test_device_plan_with_row_transform_8_per_lane(oracle, n_rot, tk, tv):
+    """The same through the 8-elements-per-lane kernel, which keeps the rotary
+    dims other than 64, 128 and 256: it reads its items, layer pointers and
+    frequencies from the plan, four layers to a workgroup."""
+    test_device_plan_with_row_transform(oracle, (n_rot, tk, tv))
