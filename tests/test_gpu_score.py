@@ -267,3 +267,60 @@ def test_score_fold_past_lds_layers(ctx, L, mode):
     if mode == kv.LAYER_MEAN:
         want = want / np.float32(L)
     assert np.array_equal(s.astype(np.float32).view(np.uint32), want.astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("D,g,Tq,T,B", [
+    (256, 6, 16, 128, 7),    # one wave of six row tiles, its keys in parts
+    (256, 6, 32, 128, 40),   # two waves
+    (256, 6, 32, 48, 40),    # two waves, tiles that span blocks
+    (256, 6, 60, 128, 24),   # four waves
+    (256, 6, 60, 16, 90),    # four waves, tiles that span blocks
+    (256, 6, 140, 128, 24),  # three slices
+    (256, 8, 100, 32, 70),   # three slices, four blocks to a tile
+    (128, 4, 20, 128, 30),
+    (128, 4, 48, 128, 30),
+    (128, 4, 48, 80, 30),
+    (128, 8, 120, 128, 30),
+])
+@pytest.mark.parametrize("at", [0.0, 0.5, 1.0])
+def test_score_bf16_past_f16_range_in_one_wave(ctx, D, g, Tq, T, B, at):
+    """One bf16 query row past f16's range: the wave that holds it loads and
+    converts its rows again, scaled, while its first key tile is under way; the
+    other waves of its workgroup and the other slices keep their scale.  Even
+    blocks have a key in the direction of that row, odd ones a key in that of
+    another row of the same KV head, and no key that the large row likes.
+    Against 64 bits of the same bf16 values: the products are exact in 32 bits
+    and their sum is within D * 2^-24 of its terms, which for the winning pair
+    add up to less than twice the sum."""
+    announce(f"bf16 past f16: D={D} g={g} Tq={Tq} T={T} B={B} rows at {at}")
+    L, Hkv = 2, 2
+    Hq, R = g * Hkv, g * Tq
+    gen = torch.Generator(device="cuda").manual_seed(D + Tq + T)
+    q = torch.randn((L, Tq, Hq, D), generator=gen, device="cuda").to(torch.bfloat16)
+    big = int(at * (R - 1))                       # one of the (token, head) rows of the first KV head
+    sign = q[:, big // g, big % g].float().sign()
+    q[:, big // g, big % g] = (sign * 7.0e4 * (1 + torch.rand((L, D), generator=gen, device="cuda"))).to(torch.bfloat16)
+    k = torch.randn((L, B, T, Hkv, D), generator=gen, device="cuda").mul_(0.01).half()
+    rng = np.random.default_rng(R)
+    for l in range(L):
+        for b in range(B):
+            r, away = big, 0.0
+            if b % 2:
+                r = (big + 1 + int(rng.integers(R - 1))) % R
+                k[l, b, :, 0] = (-0.01 * sign[l]).half()
+                # the large row times 3 d / max |d|: at most about 1.1e5 sqrt(D) rms; times
+                # the part away from it: 0.5 * 1.05e5 D on average, 5.4 times that at D = 128
+                away = 0.5 * sign[l]
+            d = q[l, r // g, r % g].float()
+            k[l, b, int(rng.integers(T)), 0] = (3.0 * d / d.abs().max() - away).half()
+    s, ls = run_score(ctx, k, q, kv.TYPE_BF16, Hq, Hkv, D, 0)
+    want = torch.full((L, B), -float("inf"), dtype=torch.float64, device="cuda")
+    for l in range(L):
+        for h in range(Hkv):
+            x = k[l, :, :, h].reshape(-1, D).double() @ q[l, :, h * g:(h + 1) * g].reshape(-1, D).double().T
+            want[l] = torch.maximum(want[l], x.view(B, -1).amax(dim=1) / D ** 0.5)
+    want = want.cpu().numpy()
+    assert want[:, ::2].min() > 1e4 and want[:, 1::2].max() < 1e4
+    tol = 2 * (D + 4) * 2.0 ** -24
+    assert np.all(np.abs(ls - want) <= tol * np.abs(want))
+    assert np.all(np.abs(s - want.mean(0)) <= 2 * tol * np.abs(want.mean(0)))
