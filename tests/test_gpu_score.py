@@ -324,3 +324,47 @@ def test_score_bf16_past_f16_range_in_one_wave(ctx, D, g, Tq, T, B, at):
     tol = 2 * (D + 4) * 2.0 ** -24
     assert np.all(np.abs(ls - want) <= tol * np.abs(want))
     assert np.all(np.abs(s - want.mean(0)) <= 2 * tol * np.abs(want.mean(0)))
+
+
+@pytest.mark.parametrize("D,g,Tq,T,last_T", [
+    (256, 6, 64, 128, 90), (256, 6, 67, 64, 50), (256, 6, 53, 128, 64), (256, 13, 16, 16, 5), (256, 7, 16, 48, 40),
+    (256, 6, 32, 128, 100), (256, 8, 100, 128, 0), (128, 4, 96, 112, 100), (128, 4, 110, 128, 3),
+    (128, 8, 29, 80, 0), (128, 4, 14, 16, 15),
+])
+def test_score_every_row_tile_decides(ctx, D, g, Tq, T, last_T):
+    """As test_score_tile_edges, with the winning row walked over the tiles of
+    16 rows, and the winning key over the groups of 16 keys: every row tile of
+    every wave and slice, in both KV heads, is some block's score."""
+    L, Hkv = 2, 2
+    Hq, R = g * Hkv, g * Tq
+    tiles, groups = (R + 15) // 16, (T + 15) // 16
+    B = max(tiles, groups) + 3
+    announce(f"scorer row tiles: D={D} g={g} Tq={Tq} T={T} last_T={last_T}: {tiles} row tiles x {groups} key groups")
+    gen = torch.Generator(device="cuda").manual_seed(D + 7 * g + 11 * Tq + T)
+    q = torch.randn((L, Tq, Hq, D), generator=gen, device="cuda").half()
+    k = torch.randn((L, B, T, Hkv, D), generator=gen, device="cuda").mul_(0.1).half()
+    nt = last_T or T
+    rng = np.random.default_rng(R + T)
+    planted = set()
+    for l in range(L):
+        for b in range(B):
+            h = (l + b // tiles) % 2
+            r = min(16 * (b % tiles) + int(rng.integers(16)), R - 1)
+            j = min(16 * (b % groups) + int(rng.integers(16)), (nt if b == B - 1 else T) - 1)
+            k[l, b, j, h] = 4 * q[l, r // g, h * g + r % g]
+            planted.add((h, r // 16))
+        if nt < T:
+            k[l, B - 1, nt:] = 40 * q[l, 0, 0]
+    assert planted >= {(h, i) for h in range(2) for i in range(tiles)}
+    s, ls = run_score(ctx, k, q, kv.TYPE_F16, Hq, Hkv, D, last_T)
+    want = torch.full((L, B), -float("inf"), dtype=torch.float64, device="cuda")
+    for l in range(L):
+        for h in range(Hkv):
+            x = k[l, :, :, h].reshape(-1, D).double() @ q[l, :, h * g:(h + 1) * g].reshape(-1, D).double().T
+            x = x.amax(dim=1).view(B, T)
+            x[B - 1, nt:] = -float("inf")
+            want[l] = torch.maximum(want[l], x.amax(dim=1) / D ** 0.5)
+    want = want.cpu().numpy()
+    tol = (D + 4) * 2.0 ** -24
+    assert np.all(np.abs(ls - want) <= tol * np.abs(want))
+    assert np.all(np.abs(s - want.mean(0)) <= 2 * tol * np.abs(want.mean(0)))
