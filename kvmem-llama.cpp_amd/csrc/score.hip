@@ -71,11 +71,13 @@ constexpr int kMaxRowTiles = 6;
 constexpr int kMaxRowWaves = 4;
 constexpr uint32_t kSliceTiles = kMaxRowTiles * kMaxRowWaves;
 constexpr uint32_t kSliceRows = kSliceTiles * 16u;
-// Below this many waves in a launch, blocks are split over key parts: 2
-// layers x 12 blocks take 8.4 us with 384 waves, 10.7 with 96; at 480 waves a
-// split already loses (12.2 against 12.7 us), to the query rows that each
-// further wave loads.
-constexpr uint32_t kSplitWaves = 256;
+// Below this many waves in a launch, blocks are split over key parts.  Mean
+// time of a call with a line at 256, 384 and 512 waves against none, over 276
+// calls of one-wave slices (2 and 4 layers, 4 to 64 blocks), by unsplit waves:
+// 96 0.85, 0.84, 0.87; 192 0.90, 0.90, 0.91; 224 0.90, 0.90, 0.97; 256 1.00,
+// 0.89, 0.90; 320 1.00, 0.93, 0.93; 384 1.00, 1.00, 0.93; 448 1.00, 1.00, 1.01.
+// Each further wave loads the query rows again.
+constexpr uint32_t kSplitWaves = 384;
 // Cache policy of the tile DMA.  Keys read by one workgroup only stream past
 // the caches (nt): L2 stays with the query rows, and the power-capped kernel
 // pays less energy (16 x 2048 blocks, 64-token query: 2.404 ms against 2.435
