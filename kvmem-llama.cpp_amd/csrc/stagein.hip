@@ -2062,9 +2062,15 @@ constexpr uint32_t kPlanThreads = 1024;
 // of neighbouring selections make about that many chains (60 segments of 256
 // selected blocks with 30 % new, 13 of 64); further segments take turns.  An
 // empty row costs the dispatch of its workgroups, a row's second segment
-// waits for the stores of its first.  Walk by rows, 30 % new blocks (us):
-//   64 selected, 16 layers of 4x256 q8_0/q4_0 (41 moves)   16: 55  32: 56  64: 62
-//   256 selected, 16 layers of 4x256 q8_0 (177 moves)      16: 309 32: 302 64: 301
+// waits for the stores of its first.  Saves and walk by rows, 16 layers of
+// 1024 elements, q8_0, 30 % of the blocks new (us; * the rule's):
+//   selected     1      4      8     16     32     64 rows
+//          8  14.2   14.3   14.2   14.3   14.3   14.3   (* 2: 14.1)
+//         16  22.6  *21.1   21.2   22.1   22.0   22.0
+//         32  39.6   38.6  *39.1   39.2   39.2   39.0
+//         64  79.1   73.9   73.8  *72.0   73.8   80.8
+//        128  89.3   86.3   84.4   82.4  *82.1   87.4
+//        256 314.2  299.3  292.8  288.2  278.7 *277.2
 constexpr uint32_t kChainRows = 64;
 constexpr uint32_t kChainRowSel = 4;  // selected blocks per row
 constexpr uint32_t kPlanMaxSel = KVMEM_PLAN_MAX_SEL;    // selected blocks per step (one per thread)
