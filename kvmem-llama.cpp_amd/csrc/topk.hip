@@ -15,10 +15,11 @@
 // digit where the running count from the top reaches the remaining rank.
 // (Scores of one call share their sign and most of their exponent.  A pass
 // over those bits puts nearly every key into one histogram word, where the
-// LDS atomics of a wave queue up.  2048 scores: 8.3 us, 10.0 with passes from
-// the top bit and four barriers each; 8192 scores: 12.7 and 21.0.  Mean cosines
-// have both signs and gain nothing: the bit is found while the keys are made,
-// and the streamed kernel looks at 1024 scores before it spends a pass on it.)
+// LDS atomics of a wave queue up.  Kernel time, and with passes from the top
+// bit and four barriers each: 2048 scores 8.4 us, 10.0; 8192 13.5, 20.7; 100000
+// 197, 279.  Mean cosines have both signs and gain nothing (2048 9.2, 9.1; 8192
+// 14.8, 14.6): the bit is found while the keys are made, and the streamed kernel
+// looks at 1024 scores before it spends a pass on it.)
 // Winners are the keys at or above that threshold; they and the forced ids are
 // compacted in ascending id order with a workgroup prefix sum, which is the
 // window order of KvMemStore::pick_topk_ungrouped (kvmem_store.cpp:618-622).
