@@ -4,8 +4,8 @@
 //
 // Producer: k_sum[l][b][e] = fp32 sum of the block's F16 keys in token
 // order, mean_tokens[l][b] = tokens summed (RawKvStore::capture_mean_f16,
-// kvmem/src/host/raw_kv_store.cpp:184-202).  A thread owns four consecutive
-// channels and adds token after token, so every channel's sum is the same
+// kvmem/src/host/raw_kv_store.cpp:184-202).  A thread owns four or eight
+// consecutive channels and adds token after token, so every channel's sum is the same
 // sequence of IEEE additions as the reference's: bit-identical.
 //
 // Scorer (llama_memory_kvmem::score_retrieval, src/adapter/
@@ -51,9 +51,15 @@ __device__ inline float add_hi(float acc, uint32_t w) {
 // blocks x 16 layers of 1024 channels (67 MB of keys): 10.6 us; 44.4 when a
 // wave waited for every row.  All of 512 blocks: 361 us = 6.0 TB/s (421).
 // Four channels per thread: eight (half the waves, each with twice the
-// additions in its chain) take 11.05 and 365 us.
+// additions in its chain) take 11.05 and 365 us.  Wide rows of blocks shorter
+// than two batches take eight: there a wave costs more than its rows (us, four
+// and eight; 16 layers x 1000 blocks of 1024 channels: 4 tokens 51.1 and 45.6,
+// 16 tokens 107 and 106, 32 tokens 194 and 195; of 2048 channels: 7 tokens 118
+// and 105; of 256 channels: 4 tokens 17.7 and 21.2).
 constexpr uint32_t kSumBatch = 16;
 constexpr int kSumChannels = 4;
+constexpr int kSumChannelsShort = 8;
+constexpr uint32_t kSumWide = 1024;
 
 template <int CH>
 __global__ __launch_bounds__(2048 / CH) void meank_sum_kernel(const uint8_t *k, uint64_t block_stride,
@@ -150,8 +156,13 @@ static void launch_meank_sum(hipStream_t stream, uint32_t jobs, const uint8_t *k
                              uint64_t layer_stride, const LaunchTables &ids, uint32_t L, uint32_t cap, uint32_t T,
                              uint32_t E, uint32_t last_block, uint32_t last_tokens, float *k_sum,
                              uint32_t *mean_tokens) {
-    meank_sum_kernel<kSumChannels><<<jobs, E / kSumChannels, 0, stream>>>(
-        k, block_stride, layer_stride, ids.dev, ids.args, L, cap, T, E, last_block, last_tokens, k_sum, mean_tokens);
+    if (E >= kSumWide && T < 2u * kSumBatch) {
+        meank_sum_kernel<kSumChannelsShort><<<jobs, E / kSumChannelsShort, 0, stream>>>(
+            k, block_stride, layer_stride, ids.dev, ids.args, L, cap, T, E, last_block, last_tokens, k_sum, mean_tokens);
+    } else {
+        meank_sum_kernel<kSumChannels><<<jobs, E / kSumChannels, 0, stream>>>(
+            k, block_stride, layer_stride, ids.dev, ids.args, L, cap, T, E, last_block, last_tokens, k_sum, mean_tokens);
+    }
 }
 
 // Query-sum producer: one thread per (layer, channel) adds the listed

@@ -498,3 +498,12 @@ def test_meank_scores_without_query_rows(ctx, nb):
     ctx.score_meank(q_sum.data_ptr(), [0, 0, 0], ks.data_ptr(), mt.data_ptr(), 3, nb, 2, 2, 128, scores.data_ptr())
     ctx.sync()
     assert not scores[:nb].any() and float(scores[nb]) == -9.0
+
+
+@pytest.mark.parametrize("n_ids", [6, 800])
+@pytest.mark.parametrize("Tb,last,E_", [(3, 1, 2048), (7, 6, 1024), (16, 0, 1032), (31, 30, 1024), (32, 31, 1024),
+                                        (20, 17, 1016)])
+def test_meank_sums_short_wide_blocks(ctx, n_ids, Tb, last, E_):
+    """The same on both sides of 1024 channels and 32 tokens, where a thread
+    takes eight channels or four."""
+    test_meank_sums_batch_edges(ctx, n_ids, Tb, last, E_)
