@@ -1655,17 +1655,31 @@ static int resolve_xf(kvmem_hip_ctx *ctx, const kvmem_hip_pool *pool, uint32_t e
     // The 64-elements-per-lane kernels hold a rotary pair in one lane (n_rot
     // 64) or in lanes l and l ^ n_rot/128 (n_rot 128, 256), and F16 rows only
     // without cross-lane butterflies (width 64); other shapes take the
-    // 8-elements-per-lane kernels.  n_rot 64 by this kernel and that one, us: 1
-    // block x 16 layers of 1024 elements 7.2 and 24.9 (F16), 24
-    // blocks, attn_rot, q8_0 65.8 and 99.5; jobs of F16 rows that fill the chip are
-    // bound by memory and up to 7 % slower here (24 layers x 33 blocks 163 and
-    // 151, 16 x 40 128 and 128.5).
+    // 8-elements-per-lane kernels (and some jobs of n_rot 64, see
+    // keep_8_per_lane).
     const uint32_t half = out.n_rot / 2;
     out.lane64 = (half == 0 || half == 32 || half == 64 || half == 128) &&
                  ek % 64 == 0 && (!want_v || ev % 64 == 0) &&
                  (pool->type_k != KVMEM_TYPE_F16 || out.had_k <= 64) &&
                  (!want_v || pool->type_v != KVMEM_TYPE_F16 || out.had_v <= 64);
     return KVMEM_HIP_OK;
+}
+
+// Whether a job of n blocks stays in the 8-elements-per-lane kernel although its
+// shape fits the other: F16 rows with 64 rotary dims and no rotation are copied
+// but for the RoPE, and a job of many layers that fills the chip is bound by
+// memory, where the walk of one workgroup over the layers is slower.  That
+// kernel and this one, us by workgroups, rows of 1024 elements: 16 layers 2048
+// 101 and 97, 4096 203 and 191, 8192 411 and 378; 24 layers 1536 130 and 118; 8
+// layers 2560 64 and 70, 4096 99 and 98, 8192 199 and 193; 12 layers 2048 76 and
+// 78, 4096 150 and 145.  Narrow rows gain nothing (16 x 200 blocks of 256
+// elements 169 and 170).
+static bool keep_8_per_lane(const kvmem_hip_pool *pool, const XfParams &xp, bool want_v, uint32_t n) {
+    const uint64_t rows = static_cast<uint64_t>(n) * pool->block_tokens;
+    const uint64_t units = rows * (pool->n_embd_k + (want_v ? pool->n_embd_v : 0u)) / (32u * kX64Groups);
+    return xp.n_rot == 64u && xp.had_k == 0 && xp.had_v == 0 && pool->type_k == KVMEM_TYPE_F16 &&
+           (!want_v || pool->type_v == KVMEM_TYPE_F16) && pool->n_embd_k >= 512u &&
+           units >= kX64FullGrid + kX64FullGrid / 2u && units * pool->n_layers >= 28u * kX64FullGrid;
 }
 
 // One upload holding a block job's device tables: the pool's per-layer
@@ -2447,6 +2461,7 @@ int kvmem_hip_stagein_blocks(kvmem_hip_ctx *ctx, const kvmem_hip_history *hist,
     if (st != KVMEM_HIP_OK) {
         return st;
     }
+    xp.lane64 = xp.lane64 && !keep_8_per_lane(pool, xp, want_v, n);
     std::vector<uint32_t> items(4 * static_cast<size_t>(n));
     for (uint32_t i = 0; i < n; ++i) {
         if (block_ids[i] >= hist->n_blocks || slots[i] >= pool->n_slots) {
@@ -2991,6 +3006,7 @@ int kvmem_hip_reselect_device_stagein(kvmem_hip_ctx *ctx, const kvmem_hip_histor
     if (xst != KVMEM_HIP_OK) {
         return xst;
     }
+    xp.lane64 = xp.lane64 && !keep_8_per_lane(pool, xp, true, n_staged);
     JobTables jt;
     jt.tables.dev = static_cast<const uint8_t *>(ctx->plan.ptr) + ctx->plan_stage_off;
     jt.items_off = 16u * L;

@@ -259,3 +259,19 @@ def test_transform_full_chip(ctx, oracle, L, B, D, hkv, n_rot, hk, tk, tv, last)
     run_case(ctx, oracle, L=L, B=B, Hkv=hkv, D=D, type_k=tk, type_v=tv, n_rot=n_rot, had_k=hk,
              had_v=64 if hk else 0, ids=rng.permutation(B).tolist(), slots=rng.permutation(B + 1)[:B].tolist(),
              n_slots=B + 1, last=last, seed=B + L)
+
+
+@pytest.mark.parametrize("L,B,D,hkv", [
+    (28, 23, 128, 8),    # 1472 units: the 64-elements-per-lane kernel
+    (28, 24, 128, 8),    # 1536 units of 28 layers: the 8-elements-per-lane one
+    (19, 48, 256, 2),    # 1536 units x 19 layers: just past its line
+    (18, 48, 256, 2),    # and before it
+])
+def test_transform_f16_rope64_large_jobs(ctx, oracle, L, B, D, hkv):
+    """F16 rows with 64 rotary dims on both sides of the line between the two
+    kernels (a smaller last block, explicit positions)."""
+    announce(f"F16, RoPE 64: {L} layers x {B} blocks of {hkv} x {D}")
+    rng = np.random.default_rng(L + B)
+    run_case(ctx, oracle, L=L, B=B, Hkv=hkv, D=D, type_k=kv.TYPE_F16, type_v=kv.TYPE_F16, n_rot=64, had_k=0,
+             had_v=0, ids=rng.permutation(B).tolist(), slots=rng.permutation(B + 1)[:B].tolist(), n_slots=B + 1,
+             last=57, pos0=rng.integers(0, 1 << 20, B).tolist(), seed=L)
