@@ -1855,14 +1855,19 @@ static int launch_block_job(kvmem_hip_ctx *ctx, int type_k, const BlockSource &k
         // A workgroup takes every layer of a unit (one cos/sin table), a wave
         // one after the other, which leaves a job of few units most of the chip
         // empty: there the layers are split over more workgroups (16 layers,
-        // RoPE 256 and attn_rot: one block 12.3 us, 35.7 unsplit).  Halves that
-        // no longer fit the chip at once still pay where they are long (8
-        // layers, attn_rot, by workgroups unsplit: 576 17.6 and 19.7, 704 20.2
-        // and 20.5, 832 23.1 and 22.1; 24 layers: 832 55.0 and 58.8, 960 61.4
-        // and 62.1).
-        while (sk.layer_group > 4u && grid() * sk.layer_group <= uint64_t{kX64FullGrid} * (sk.layer_group - 2u)) {
-            sk.layer_group = ((sk.layer_group + 1u) / 2u + 3u) / 4u * 4u;
-            sv_copy.layer_group = sk.layer_group;
+        // RoPE 256 and attn_rot: one block 12.3 us, 35.7 unsplit).  Up to 12
+        // layers are not worth more than 1536 workgroups, one and a half times
+        // what the chip holds at once (attn_rot, us by workgroups, split and
+        // not: 8 layers 1152 17.6 and 19.7, 1408 20.2 and 20.5, 1664 23.1 and
+        // 22.1; 12 layers 1920 35.7 and 32.8; but 16 layers 1664 38.9 and 40.8,
+        // 24 layers 1920 61.4 and 62.1).
+        const uint64_t unsplit = grid();
+        while (sk.layer_group > 4u && grid() < kX64FullGrid) {
+            const uint32_t lg = ((sk.layer_group + 1u) / 2u + 3u) / 4u * 4u;
+            if (sk.layer_group <= 12u && 2u * unsplit * ((sk.n_layers + lg - 1u) / lg) > 3u * kX64FullGrid) {
+                break;
+            }
+            sk.layer_group = sv_copy.layer_group = lg;
         }
     }
     const uint64_t nk = block_job_chunks(sk, n_items);

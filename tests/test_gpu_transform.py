@@ -275,3 +275,17 @@ def test_transform_f16_rope64_large_jobs(ctx, oracle, L, B, D, hkv):
     run_case(ctx, oracle, L=L, B=B, Hkv=hkv, D=D, type_k=kv.TYPE_F16, type_v=kv.TYPE_F16, n_rot=64, had_k=0,
              had_v=0, ids=rng.permutation(B).tolist(), slots=rng.permutation(B + 1)[:B].tolist(), n_slots=B + 1,
              last=57, pos0=rng.integers(0, 1 << 20, B).tolist(), seed=L)
+
+
+@pytest.mark.parametrize("L,B,tk", [
+    (12, 25, kv.TYPE_Q8_0),  # parts of 4 layers, by way of 8 + 4
+    (10, 44, kv.TYPE_Q5_0),  # parts of 8 and 2
+    (8, 52, kv.TYPE_Q4_0),   # one part: two would be 1664 workgroups
+])
+def test_transform_layer_parts(ctx, oracle, L, B, tk):
+    """Layer splits of jobs of 400 to 832 workgroups: 4 + 4 + 4, 8 + 2, none."""
+    announce(f"{L} layers x {B} blocks, K={tk}")
+    rng = np.random.default_rng(B)
+    run_case(ctx, oracle, L=L, B=B, Hkv=2, D=128, type_k=tk, type_v=kv.TYPE_Q8_0, n_rot=64, had_k=128, had_v=64,
+             ids=rng.permutation(B).tolist(), slots=rng.permutation(B + 1)[:B].tolist(), n_slots=B + 1, last=41,
+             seed=L)
